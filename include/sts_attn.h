@@ -437,8 +437,11 @@ int sts_q4k_dequant(const uint8_t* weights, float* out, uint32_t k, uint32_t n, 
  * product for more than one row, which the reference runs with the
  * one-thread-per-output shader (q4k_matmul with M > 1, gguf.rs:810-897 and
  * wgsl/shader_q4k.wgsl; q4k_matmul_with_residual, gguf.rs:899-905).  The
- * weights are dequantised exactly as the shader rounds them and multiplied
- * in f32 on the matrix cores.  With swiglu != 0 the matrix has n = 2F rows and
+ * products run on the bf16 matrix cores with every f32 x as the exact sum of
+ * three bf16 values and the quants as they are, accumulated and scaled in
+ * f32: no operand is rounded, and the result is as close to the exact product
+ * as with f32 matrix instructions on the dequantised weights.  With
+ * swiglu != 0 the matrix has n = 2F rows and
  * y[m][j] = silu(G[m][j]) * G[m][j + F] for j < F (the SwiGLU of
  * wgsl/shader_swiglu.wgsl applied to the product; residual must be NULL).
  * With norm_alpha non-NULL each x row is first RMS-normalised,
@@ -446,9 +449,7 @@ int sts_q4k_dequant(const uint8_t* weights, float* out, uint32_t k, uint32_t n, 
  * every projection of the depformer, depth_engine.rs:1069-1095, 1262-1282,
  * fused; its sum of squares is taken in this kernel's order, not the
  * shader's).  k must be a multiple of 256 in 256..16384; above 4096 (the
- * temporal FFN's linear_out, k = 11264) the product runs as slices of 4096
- * summed in slice order by a second kernel, through the stream's library
- * workspace (see the workspace rules above), without norm_alpha or swiglu.
+ * temporal FFN's linear_out, k = 11264) without norm_alpha or swiglu.
  * x rows, norm_alpha and weights 16-byte aligned; ldx, ldy, ldr are row
  * strides in floats (ldx a multiple of 4).
  */

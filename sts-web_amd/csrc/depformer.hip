@@ -5,20 +5,8 @@
 // Q4_K matvecs, cache writes, attention, SwiGLU and residual adds, then an
 // output matvec and top-k sampling, each a separate WGSL dispatch.  Here the
 // streams of a batch share every weight read: the Q4_K products become
-// GEMMs with the streams as the M dimension.
-//
-// q4k_gemm_kernel.  Workgroup = one 16-stream tile x all K: wave kb owns
-// super-block column kb (256 weights of every row) and keeps the 64 x values
-// of its lane in registers; the workgroup walks 16-row tiles.  Per tile a
-// wave dequantises the shader's f32 weights w = (d*scale)*q - dmin*min
-// (shader_q4k_matvec.wgsl:117-136, products and difference rounded
-// separately, so the weights are bit-identical) and feeds them to
-// v_mfma_f32_16x16x4f32: lane (r, g) supplies W[n0 + r][k] and X[m0 + r][k]
-// for k = 256 kb + 64 g + i at instruction i, g = lane / 16 being slot g of
-// the super-block (its 32 quant bytes, low nibbles sub-block 2g, high 2g+1).
-// The waves' partial tiles are summed through LDS in wave order
-// (deterministic), with the residual or the SwiGLU of a gate/value row pair
-// applied on the way out.
+// GEMMs with the streams as the M dimension.  The Q4_K GEMM is in
+// q4k_gemm.hip; here are the RMSNorm, the embedding and the sampler.
 #include <algorithm>
 #include <cfloat>
 #include <cstdint>
@@ -31,214 +19,6 @@
 namespace sts {
 
 namespace {
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kGemmBufferWord3 = 0x00020000;  // raw 32-bit buffer, no swizzle
-
-__device__ __forceinline__ u32x4 ld16(const uint8_t* p) {
-  return *reinterpret_cast<const u32x4*>(p);
-}
-
-// The 48 weight bytes lane (r, g) needs of one super-block row: header and
-// the 32 quant bytes of slot g.
-struct WTile {
-  u32x4 hd, qa, qb;
-};
-
-// MAXT: the largest workgroup (64 * K/256 threads) the instance runs with;
-// 256 (K <= 1024) leaves the register file to the prefetch buffers.  Three
-// waves per SIMD (three 4-wave workgroups per CU at K <= 1024): one register
-// past 168 would leave room for two.
-template <bool SWIGLU, int MAXT>
-__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(3)))
-void q4k_gemm_kernel(const Q4kGemmParams p) {
-#pragma clang fp contract(off)
-  constexpr int NH = SWIGLU ? 2 : 1;
-  __shared__ float part[16][NH][256];
-  __shared__ float ssq[16][16];
-  __shared__ float s_inv[16];  // 1/rms of the tile's rows (RMSNorm)
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int kb = tid >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const uint32_t KB = p.K / kQ4kBlockWeights;  // waves in the workgroup
-  const uint32_t z = blockIdx.z, mt = blockIdx.y;
-  const uint8_t* W = p.w[z];
-  const float* X = p.x + z * p.x_zstride;
-  float* Y = p.y + z * p.y_zstride;
-  const uint32_t nout = SWIGLU ? p.swiglu_f : p.N;
-  const uint32_t ntiles = (nout + 15) / 16;
-  const size_t row_bytes = (size_t)(p.w_row_blocks ? p.w_row_blocks : KB) * kQ4kBlockBytes;
-
-  // Rows past the end (and tiles past the last) re-read valid rows; their
-  // outputs are not stored.
-  auto load_w = [&](WTile (&wt)[NH], uint32_t t) {
-    t = min(t, ntiles - 1);
-#pragma unroll
-    for (int hv = 0; hv < NH; ++hv) {
-      const uint32_t n = min(t * 16 + r + (hv ? p.swiglu_f : 0u), p.N - 1);
-      const uint8_t* blk = W + n * row_bytes + (size_t)kb * kQ4kBlockBytes;
-      wt[hv].hd = ld16(blk);
-      wt[hv].qa = ld16(blk + 16 + 32 * g);
-      wt[hv].qb = ld16(blk + 32 + 32 * g);
-    }
-  };
-  // The first tile's weights are requested before x, so both latencies overlap.
-  WTile cur[NH], nxt[NH];
-  load_w(cur, blockIdx.x);
-
-  // x values of this lane: X[m][256 kb + 64 g + j], j < 64 (zero past M).
-  // The tile's rows come in through a buffer resource that ends with its last
-  // row inside M, so rows past M read zeros: no per-row branch or select.
-  const uint32_t rows_here = min(16u, p.M - mt * 16);
-  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(X) + (size_t)mt * 16 * p.ldx, 0,
-      (int)(((uint64_t)(rows_here - 1) * p.ldx + p.K) * sizeof(float)), kGemmBufferWord3);
-  auto ldx4 = [&](uint32_t row, uint32_t col) {
-    return __builtin_bit_cast(
-        float4, __builtin_amdgcn_raw_buffer_load_b128(
-                    xrs, (uint32_t)((row * p.ldx + col) * sizeof(float)), 0, 0));
-  };
-  float xv[64];
-  {
-    // Through a per-wave LDS chunk (16 rows x 64 floats, pitch 68) so the
-    // global loads are coalesced: instruction i of chunk c reads rows
-    // 4i..4i+3, 256 contiguous bytes each; the lanes of slot g then copy
-    // chunk g (the 16 lanes of a read phase hit distinct banks).  (Each lane
-    // reading its own 256 bytes would touch 64 cache lines per instruction.)
-    // Chunks in flight at once: all four where a wave may hold 168 registers,
-    // two in the 16-wave instance (128).
-    constexpr int CIF = MAXT <= 256 ? 4 : 2;
-    __shared__ __align__(16) float xs[MAXT / 64][16][68];
-#pragma unroll
-    for (int c0 = 0; c0 < 4; c0 += CIF) {
-      float4 ld[CIF][4];
-#pragma unroll
-      for (int c = 0; c < CIF; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          ld[c][i] = ldx4(4 * i + (lane >> 4), 256 * kb + 64 * (c0 + c) + 4 * (lane & 15));
-#pragma unroll
-      for (int c = 0; c < CIF; ++c) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<float4*>(&xs[kb][4 * i + (lane >> 4)][4 * (lane & 15)]) = ld[c][i];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (g == c0 + c) {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const float4 t = *reinterpret_cast<const float4*>(&xs[kb][r][4 * j]);
-            xv[4 * j] = t.x;
-            xv[4 * j + 1] = t.y;
-            xv[4 * j + 2] = t.z;
-            xv[4 * j + 3] = t.w;
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-    }
-  }
-  if (p.norm_alpha) {
-    // RMSNorm of the 16 rows (shader_rmsnorm.wgsl:80-90), x * (1/rms) * alpha,
-    // with the sum of squares taken over this workgroup's registers.  alpha
-    // scales x here and 1/rms (one factor per row) scales the row's outputs
-    // in the epilogue: sum_k w (x alpha) / rms, one multiply per x value
-    // instead of two.
-    float q = 0.f;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) q = __builtin_fmaf(xv[j], xv[j], q);
-    q += __shfl_xor(q, 16, 64);
-    q += __shfl_xor(q, 32, 64);
-    if (g == 0) ssq[kb][r] = q;
-    __syncthreads();
-    if (tid < 16) {
-      float tot = ssq[0][tid];
-      for (uint32_t w = 1; w < KB; ++w) tot += ssq[w][tid];
-      s_inv[tid] = 1.0f / sqrtf(tot / (float)p.K + p.norm_eps);
-    }
-    const float4* al = reinterpret_cast<const float4*>(p.norm_alpha + 256 * kb + 64 * g);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float4 a = al[j];
-      xv[4 * j] = xv[4 * j] * a.x;
-      xv[4 * j + 1] = xv[4 * j + 1] * a.y;
-      xv[4 * j + 2] = xv[4 * j + 2] * a.z;
-      xv[4 * j + 3] = xv[4 * j + 3] * a.w;
-    }
-  }
-
-  for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    // The next tile's weights are in flight during this one (the condition
-    // is uniform over the workgroup).
-    if (t + gridDim.x < ntiles) load_w(nxt, t + gridDim.x);
-#pragma unroll
-    for (int hv = 0; hv < NH; ++hv) {
-      const u32x4 hd = cur[hv].hd, qa = cur[hv].qa, qb = cur[hv].qb;
-      const float d = half_bits_to_float(hd.x), dmin = half_bits_to_float(hd.x >> 16);
-      uint32_t scl, mnl, sch, mnh;
-      scale_min(hd.y, hd.z, hd.w, 2 * g, scl, mnl);
-      scale_min(hd.y, hd.z, hd.w, 2 * g + 1, sch, mnh);
-      // d1 = d*scale and m1 = dmin*min are exact in f32 (11-bit f16
-      // significands times 6-bit integers), and so is q*d1 (4-bit q), so
-      // fma(q, d1, -m1) rounds once, where the shader's (d*scale)*q - dmin*min
-      // rounds: the same weight, bit for bit.
-      const float d1 = d * (float)scl, m1 = dmin * (float)mnl;
-      const float d2 = d * (float)sch, m2 = dmin * (float)mnh;
-      const uint32_t words[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-      floatx4 acc[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        uint32_t lo = words[w] & 0x0F0F0F0Fu;
-        uint32_t hi = (words[w] >> 4) & 0x0F0F0F0Fu;
-        // Opaque to the optimiser, so each byte below is one v_cvt_f32_ubyte.
-        asm("" : "+v"(lo), "+v"(hi));
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float wl = __builtin_fmaf((float)((lo >> (8 * b)) & 0xFFu), d1, -m1);
-          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wl, xv[4 * w + b], acc[b], 0, 0, 0);
-        }
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float wh = __builtin_fmaf((float)((hi >> (8 * b)) & 0xFFu), d2, -m2);
-          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wh, xv[32 + 4 * w + b], acc[b], 0, 0, 0);
-        }
-      }
-      const floatx4 s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-      // Accumulator element e of lane (r, g) is row 4g + e, stream r of the tile.
-#pragma unroll
-      for (int e = 0; e < 4; ++e) part[kb][hv][(4 * g + e) * 16 + r] = s[e];
-    }
-    __syncthreads();
-    for (int o = tid; o < 256; o += blockDim.x) {
-      const uint32_t mo = mt * 16 + (o & 15), no = t * 16 + (o >> 4);
-      float v = part[0][0][o];
-      for (uint32_t w = 1; w < KB; ++w) v += part[w][0][o];
-      const float inv = p.norm_alpha ? s_inv[o & 15] : 1.0f;
-      v *= inv;
-      if constexpr (SWIGLU) {
-        float u = part[0][NH - 1][o];
-        for (uint32_t w = 1; w < KB; ++w) u += part[w][NH - 1][o];
-        u *= inv;
-        v = v / (1.0f + expf(-v)) * u;
-      }
-      if (mo < p.M && no < nout) {
-        if (p.res) v += p.res[(size_t)mo * p.ldr + no];
-        Y[(size_t)mo * p.ldy + no] = v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int hv = 0; hv < NH; ++hv) cur[hv] = nxt[hv];
-  }
-}
 
 // One workgroup of 256 per row, shader_rmsnorm.wgsl:27-92 step for step.
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ x,
@@ -844,95 +624,7 @@ __global__ __launch_bounds__(256) void sample_topk_kernel(const SampleParams p) 
   if (tid == pick) *outp = slot_idx[0xFFFFFFFFu - (uint32_t)key];
 }
 
-// y[m][n] = sum over the slices s of part[s][m][n] in slice order, plus
-// res[m][n]: the split-K sum of launch_q4k_gemm.
-__global__ __launch_bounds__(256) void splitk_sum_kernel(const float* __restrict__ part,
-                                                         uint32_t nsl, uint32_t M, uint32_t N,
-                                                         const float* __restrict__ res,
-                                                         uint64_t ldr, float* __restrict__ y,
-                                                         uint64_t ldy) {
-#pragma clang fp contract(off)
-  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (uint64_t)M * N) return;
-  const uint32_t m = (uint32_t)(i / N), n = (uint32_t)(i % N);
-  float v = part[i];
-  for (uint32_t s = 1; s < nsl; ++s) v += part[(uint64_t)s * M * N + i];
-  if (res) v += res[(size_t)m * ldr + n];
-  y[(size_t)m * ldy + n] = v;
-}
-
 }  // namespace
-
-int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
-  // Every check runs before anything is allocated or launched.
-  if (p.K % kQ4kBlockWeights != 0 || p.K == 0 || p.K > 64 * kQ4kBlockWeights)
-    return fail(STS_ERR_INVALID, "GEMM K = %u must be a multiple of 256 in 256..16384", p.K);
-  if (p.M == 0 || p.N == 0 || p.Z == 0 || p.Z > (uint32_t)kGemmMaxZ)
-    return fail(STS_ERR_INVALID, "GEMM shape M=%u N=%u Z=%u", p.M, p.N, p.Z);
-  if ((p.M + 15) / 16 > 65535u) return fail(STS_ERR_INVALID, "M = %u too large", p.M);
-  if (p.swiglu_f && (p.swiglu_f * 2 != p.N))
-    return fail(STS_ERR_INVALID, "SwiGLU GEMM needs N = 2F (N=%u F=%u)", p.N, p.swiglu_f);
-  if (p.ldx % 4 != 0 || p.x_zstride % 4 != 0 || (reinterpret_cast<uintptr_t>(p.x) & 15))
-    return fail(STS_ERR_INVALID, "GEMM x rows must be 16-byte aligned");
-  // A 16-row tile of x is addressed through one buffer resource (31-bit range).
-  if ((uint64_t)p.ldx * 15 * sizeof(float) + (uint64_t)p.K * sizeof(float) > 0x7FFFFFF0ull)
-    return fail(STS_ERR_INVALID, "GEMM x row stride %llu too large",
-                (unsigned long long)p.ldx);
-  for (uint32_t z = 0; z < p.Z; ++z)
-    if (!p.w[z] || (reinterpret_cast<uintptr_t>(p.w[z]) & 15))
-      return fail(STS_ERR_INVALID, "GEMM weights %u null or not 16-byte aligned", z);
-  if (p.K > 16 * kQ4kBlockWeights) {
-    // Split K: slices of up to 16 super-blocks into a workspace, then the sum.
-    if (p.Z != 1 || p.swiglu_f || p.norm_alpha)
-      return fail(STS_ERR_INVALID, "GEMM with K = %u > 4096 takes no SwiGLU, RMSNorm or Z > 1",
-                  p.K);
-    const uint32_t KB = p.K / kQ4kBlockWeights;
-    const uint32_t nsl = (KB + 15) / 16;
-    const size_t mn = (size_t)p.M * p.N;
-    const uint64_t blocks = (mn + 255) / 256;
-    if (blocks > 0x7FFFFFFFull) return fail(STS_ERR_INVALID, "GEMM M x N = %zu too large", mn);
-    Workspace* ws = nullptr;
-    if (int rc = get_workspace(stream, nsl * mn, 0, &ws)) return rc;
-    for (uint32_t sl = 0; sl < nsl; ++sl) {
-      const uint32_t kb0 = sl * 16, kbs = std::min(16u, KB - kb0);
-      Q4kGemmParams q = p;
-      q.w[0] = p.w[0] + (size_t)kb0 * kQ4kBlockBytes;
-      q.x = p.x + (size_t)kb0 * kQ4kBlockWeights;
-      q.K = kbs * kQ4kBlockWeights;
-      q.w_row_blocks = KB;
-      q.res = nullptr;
-      q.y = ws->part + sl * mn;
-      q.ldy = p.N;
-      if (int rc = launch_q4k_gemm(q, stream)) return rc;
-    }
-    hipLaunchKernelGGL(splitk_sum_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream,
-                       ws->part, nsl, p.M, p.N, p.res, p.ldr, p.y, p.ldy);
-    STS_HIP(hipGetLastError());
-    return STS_OK;
-  }
-  const uint32_t KB = p.K / kQ4kBlockWeights;
-  const uint32_t mtiles = (p.M + 15) / 16;
-  const uint32_t nout = p.swiglu_f ? p.swiglu_f : p.N;
-  const uint32_t ntiles = (nout + 15) / 16;
-  // Up to 4 workgroups per CU in total; each walks ntiles / gx row tiles and
-  // reads its 16 x rows once.
-  const uint32_t cus = (uint32_t)device_cu_count();
-  const uint32_t gx = std::max(1u, std::min(ntiles, 4 * cus / std::max(1u, mtiles * p.Z)));
-  const dim3 grid(gx, mtiles, p.Z), block(64 * KB);
-  if (KB <= 4) {
-    if (p.swiglu_f)
-      hipLaunchKernelGGL((q4k_gemm_kernel<true, 256>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((q4k_gemm_kernel<false, 256>), grid, block, 0, stream, p);
-  } else {
-    if (p.swiglu_f)
-      hipLaunchKernelGGL((q4k_gemm_kernel<true, 1024>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((q4k_gemm_kernel<false, 1024>), grid, block, 0, stream, p);
-  }
-  STS_HIP(hipGetLastError());
-  return STS_OK;
-}
 
 int launch_rmsnorm(const float* x, const float* alpha, float* out, uint32_t rows, uint32_t D,
                    float eps, hipStream_t stream) {

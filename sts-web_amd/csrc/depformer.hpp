@@ -1,5 +1,5 @@
 // depformer.hpp -- the depformer step chain (crates/sts-wasm/src/depth_engine.rs:884-1491)
-// batched over streams: Q4_K GEMM on f32 MFMA, RMSNorm, embedding + add, top-k sampling.
+// batched over streams: Q4_K GEMM, RMSNorm, embedding + add, top-k sampling.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -32,14 +32,8 @@ struct Q4kGemmParams {
   // the row's 1/rms to its outputs.
   const float* norm_alpha = nullptr;
   float norm_eps = 0.f;
-  // Super-blocks per weight row when the launch covers only part of K (a
-  // split-K slice of a wider matrix); 0: K / 256.
-  uint32_t w_row_blocks = 0;
 };
-// K above 4096 (no RMSNorm or SwiGLU, Z = 1) runs as ceil(K / 4096) slices
-// into a stream workspace, summed in slice order by a second kernel that also
-// adds the residual: deterministic, and refused while the stream is being
-// captured if the workspace has to grow.
+// K above 4096 takes no RMSNorm or SwiGLU and Z = 1 only.  (q4k_gemm.hip)
 int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream);
 
 // out[b][i] = x[b][i] * (1 / sqrt(sum x^2 / D + eps)) * alpha[i] in the
