@@ -450,6 +450,9 @@ int sts_q4k_dequant(const uint8_t* weights, float* out, uint32_t k, uint32_t n, 
  * fused; its sum of squares is taken in this kernel's order, not the
  * shader's).  k must be a multiple of 256 in 256..16384; above 4096 (the
  * temporal FFN's linear_out, k = 11264) without norm_alpha or swiglu.
+ * Large products (from 33 rows) keep x's operands in the stream's library
+ * workspace (at most 1024 rows' at a time); where that would have to grow while
+ * the stream is being captured, the call runs without it.
  * x rows, norm_alpha and weights 16-byte aligned; ldx, ldy, ldr are row
  * strides in floats (ldx a multiple of 4).
  */

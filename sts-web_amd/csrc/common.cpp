@@ -86,6 +86,19 @@ int get_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Wor
   return STS_OK;
 }
 
+int try_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Workspace** out) {
+  *out = nullptr;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  STS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const int rc = get_workspace(stream, part_floats, n_counters, out);
+  STS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  if (rc != STS_ERR_STATE && rc != STS_ERR_NOMEM) return rc;
+  *out = nullptr;
+  (void)hipGetLastError();
+  clear_error();
+  return STS_OK;
+}
+
 namespace {
 std::atomic<uint32_t> g_wait_limit{1u << 24};
 }  // namespace

@@ -47,6 +47,12 @@ struct Workspace {
 // when it would have to allocate while the stream is being captured.
 int get_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Workspace** out);
 
+// get_workspace for callers that have another way: *out stays null, with
+// STS_OK, where the workspace would have to grow and cannot (`stream` is being
+// captured, memory is short).  The allocation is made in relaxed capture mode,
+// so that it does not break a capture of another stream in progress.
+int try_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Workspace** out);
+
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
 

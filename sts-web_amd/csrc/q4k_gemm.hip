@@ -46,10 +46,6 @@ constexpr uint32_t kSkip = 0x80000000u;       // buffer offset past every resour
 __device__ __forceinline__ u32x4 ld16(const uint8_t* p) {
   return *reinterpret_cast<const u32x4*>(p);
 }
-__device__ __forceinline__ u32x2 ld8(const uint8_t* p) {
-  return *reinterpret_cast<const u32x2*>(p);
-}
-
 // Two of the four nibbles (one per byte of w, each 0..15) as bf16: byte q is
 // the FP8 E4M3 number q * 2^-9 (subnormal below 8), so the conversion scaled
 // by 2^9 gives q exactly.
@@ -91,6 +87,11 @@ __device__ __forceinline__ Split3 split3(const float (&x)[8]) {
   return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m),
           __builtin_bit_cast(bf16x8, l)};
 }
+
+// The value is computed here: without this the compiler puts off the
+// additions of unrolled steps to their end and keeps every step's products in
+// registers until then.
+__device__ __forceinline__ void pin(floatx4& v) { asm volatile("" : "+v"(v)); }
 
 // The products of hi, and those of lo and mid, summed apart and then added.
 template <typename F>
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
         for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(s[j][e], d1, t[e]);
       }
       acc[i] += t;
-      __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time in registers
+      pin(acc[i]);  // one tile's operands at a time in registers
     }
   }
 
@@ -357,6 +358,376 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
   }
 }
 
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// Many rows.  Here the matrix core's share is large enough for the scaling of
+// every sub-block's sum in f32 (four additions a tile and lane) to cost more
+// than it, so the 6-bit scales go into the weight operand: sc*(q - 8) is a
+// whole number up to 504, exact in f16, and d alone is left for the super-block's
+// sum.  x then has to be f16 too: the 256 values of a row and super-block are
+// scaled by a power of two that brings the largest to 2^14..2^15 and split
+// into kParts f16 values, each the rest rounded to nearest (two parts hold 22
+// bits and the sign of the rest, three all 24, both down to 2^-39 of the
+// largest).  The mins, (dmin*mn - 8*d*sc) times the sub-block's sum of x, go
+// through v_mfma_f32_16x16x4f32 as in q4k_rows_kernel.
+constexpr int kParts = 2;
+constexpr int kTileM = 64, kTileN = 128;
+
+// What split_planes_kernel writes for `rows` rows (a multiple of 64) of K
+// columns, in floats: operand units of 64 x 16 bytes per (16-row tile mt,
+// sub-block kb, part), entry g*16 + r being row r, columns 8g..8g+7, as lane
+// (r, g) of a matrix instruction wants it; the sums of x per (mt, kb, row);
+// and the inverse scales per (mt, super-block, row).
+struct TilePlanes {
+  u32x4* units;
+  float* sums;
+  float* scales;
+  static size_t floats(size_t rows, size_t KB) {
+    return rows / 16 * KB * kParts * 256 + rows * KB + rows * (KB / 8);
+  }
+  TilePlanes(float* p, size_t rows, size_t KB)
+      : units(reinterpret_cast<u32x4*>(p)),
+        sums(p + rows / 16 * KB * kParts * 256),
+        scales(sums + rows * KB) {}
+};
+
+// One wave per 16-row tile and super-block: lane (r, g) takes row r, columns
+// 8g..8g+7 of each of the eight sub-blocks.  Rows past M become zeros.  The
+// sums of x are taken in f64 and rounded once.
+__global__ __launch_bounds__(256) void split_planes_kernel(const float* __restrict__ x,
+                                                           uint64_t ldx, uint32_t M, uint32_t SB,
+                                                           u32x4* __restrict__ units,
+                                                           float* __restrict__ sums,
+                                                           float* __restrict__ scales) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, g = lane >> 4;
+  const uint32_t sb = blockIdx.x * 4 + (threadIdx.x >> 6), mt = blockIdx.y;
+  if (sb >= SB) return;
+  const uint32_t m = mt * 16 + r;
+  const float* row = x + (size_t)(m < M ? m : 0) * ldx + 256 * (size_t)sb + 8 * g;
+  float v[8][8];
+  float big = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float4 a = *reinterpret_cast<const float4*>(row + 32 * j);
+    const float4 b = *reinterpret_cast<const float4*>(row + 32 * j + 4);
+    const float t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[j][e] = m < M ? t[e] : 0.f;
+      big = fmaxf(big, fabsf(v[j][e]));
+    }
+  }
+  big = max_xor32(max_xor16(big));
+  // 2^(14 - e) for the largest value's exponent e, inside f32's normal range
+  // (an infinity or NaN passes through unscaled or not and makes the row's
+  // outputs so, which then take row_dot).
+  int e = (int)(__float_as_uint(big) >> 23) - 127;
+  e = max(-110, min(e, 127));
+  const float up = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
+  if (g == 0)
+    scales[((size_t)mt * SB + sb) * 16 + r] = __uint_as_float((uint32_t)(127 - 14 + e) << 23);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const size_t kb = (size_t)mt * SB * 8 + 8 * sb + j;
+    u32x4* u = units + kb * kParts * 64 + (g * 16 + r);
+    float rest[8];
+    double q = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      rest[i] = v[j][i] * up;
+      q += (double)v[j][i];
+    }
+#pragma unroll
+    for (int c = 0; c < kParts; ++c) {
+      f16x8 h;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        h[i] = (_Float16)rest[i];
+        rest[i] -= (float)h[i];
+      }
+      u[64 * c] = __builtin_bit_cast(u32x4, h);
+    }
+    q += __shfl_xor(q, 16, 64);
+    q += __shfl_xor(q, 32, 64);
+    if (g == 0) sums[kb * 16 + r] = (float)q;
+  }
+}
+
+// q4k_tile_kernel: many rows, the x operands prepared by split_planes_kernel.
+// Workgroup = 64 rows x 128 weight rows, four waves of 64 x 32 (4 x 2 tiles of
+// 16 x 16), two workgroups a CU, a range of super-blocks of K in steps of 64
+// columns (32 quant bytes of every weight row: two sub-blocks).  Operands go to
+// LDS through registers, two buffers each: a step's x operands
+// one step ahead, a super-block's weight bytes
+// (128 x 144) come in two batches during the super-block before.  The
+// super-block's products accumulate in the matrix core, those of
+// the first part and of the others apart (the others' sums are small, so that
+// only the first part's eight additions round at the size of the result); then
+// they are scaled by d and the row's scale and added to the total.
+struct Q4kTileParams {
+  const uint8_t* w;
+  const u32x4* units;
+  const float* sums;
+  const float* scales;
+  const float* x;  // the rows themselves, for outputs that are not finite
+  const float* res;
+  float* y;
+  uint64_t ldx, ldr, ldy, y_split;  // y_split: floats from one K range's y to the next
+  uint32_t M, N, K, mtiles, ksplit;  // mtiles: 64-row tiles
+};
+
+// Waits for this wave's LDS operations alone, then the workgroup barrier:
+// loads into registers stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Weight operand of one sub-block: the eight values sc*(q - 8), q the high
+// nibbles of w's bytes.  The half 0x5400 | 16 q is 64 + q, so one fma per pair,
+// (64 + q) sc - 72 sc, gives it exactly (72 sc = 9 sc * 8 fits 11 bits).
+__device__ __forceinline__ f16x8 weights_f16(u32x2 w, _Float16 sc, _Float16 sc72) {
+  const f16x2 s = {sc, sc}, t = {sc72, sc72};
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t h = __builtin_amdgcn_perm(0x54545454u, (i & 2 ? w.y : w.x) & 0xF0F0F0F0u,
+                                             i & 1 ? 0x04030402u : 0x04010400u);
+    o[i] = __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, h), s, -t));
+  }
+  return __builtin_bit_cast(f16x8, o);
+}
+
+__global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p) {
+#pragma clang fp contract(off)
+  __shared__ u32x4 xb[2][4][2][kParts][64];  // buffer, 16-row tile, sub-block, part
+  __shared__ u32x4 wb[2][kTileN * 9];        // buffer, weight row's super-block
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  // Workgroups are dealt to the eight XCDs round robin: all row tiles of a
+  // weight block run on one XCD, next to each other, and share its L2.
+  const uint32_t nblocks = (p.N + kTileN - 1) / kTileN;
+  const uint32_t local = blockIdx.x >> 3;
+  const uint32_t nz = local / p.mtiles * 8 + (blockIdx.x & 7u), mb = local % p.mtiles;
+  if (nz >= nblocks * p.ksplit) return;
+  const uint32_t nb = nz % nblocks, z = nz / nblocks;
+  const uint32_t KB = p.K / 32, SB = p.K / kQ4kBlockWeights;
+  const uint32_t sb0 = z * SB / p.ksplit, sb1 = (z + 1) * SB / p.ksplit;
+  const size_t row_bytes = (size_t)SB * kQ4kBlockBytes;
+
+  // x: wave w stages 16-row tile w, contiguous in memory and in LDS.
+  constexpr int XU = 2 * kParts;
+  const u32x4* xsrc = p.units + (size_t)(mb * 4 + wave) * KB * kParts * 64 + lane;
+  auto load_x = [&](u32x4 (&d)[XU], uint32_t s) {
+#pragma unroll
+    for (int u = 0; u < XU; ++u) d[u] = xsrc[(size_t)s * (XU * 64) + 64 * u];
+  };
+  auto put_x = [&](int b, const u32x4 (&d)[XU]) {
+#pragma unroll
+    for (int u = 0; u < XU; ++u) xb[b][wave][u / kParts][u % kParts][lane] = d[u];
+  };
+  // Weights: 1152 entries of 16 bytes, entry i being bytes 16 (i % 9) .. of
+  // weight row i / 9; thread t moves entries t, t + 256, ..., the last half
+  // round entry 1151 once more.  Rows past the last re-read it.
+  constexpr int WE = kTileN * 9, WU = (WE + 255) / 256;
+  uint32_t wsrc[WU], wdst[WU];
+  const uint32_t nfirst = nb * kTileN;
+#pragma unroll
+  for (int k = 0; k < WU; ++k) {
+    wdst[k] = min((uint32_t)tid + 256 * k, (uint32_t)WE - 1);
+    wsrc[k] = (min(nfirst + wdst[k] / 9, p.N - 1) - nfirst) * (uint32_t)row_bytes + 16 * (wdst[k] % 9);
+  }
+  const uint8_t* wrow0 = p.w + (size_t)nfirst * row_bytes;
+  // In two batches, entries 0-1 and 2-4 of each thread.
+  auto load_w = [&](u32x4 (&d)[3], int batch, uint32_t sb) {
+    const uint8_t* src = wrow0 + (size_t)sb * kQ4kBlockBytes;
+#pragma unroll
+    for (int k = 0; k < 2 + batch; ++k) d[k] = ld16(src + wsrc[2 * batch + k]);
+  };
+  auto put_w = [&](uint32_t b, const u32x4 (&d)[3], int batch) {
+#pragma unroll
+    for (int k = 0; k < 2 + batch; ++k) wb[b][wdst[2 * batch + k]] = d[k];
+  };
+  // Per super-block: row sums for the min product (row r of tile t, sub-block
+  // g of each half) and the inverse scales of rows 4g .. 4g+3.
+  const float* sxsrc = p.sums + (size_t)mb * 4 * KB * 16 + g * 16 + r;
+  const float* scsrc = p.scales + (size_t)mb * 4 * SB * 16 + 4 * g;
+  auto load_sx = [&](float (&d)[4][2], uint32_t sb) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) d[t][hf] = sxsrc[((size_t)t * KB + 8 * sb + 4 * hf) * 16];
+  };
+  auto load_scale = [&](floatx4 (&d)[4], uint32_t sb) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      d[t] = *reinterpret_cast<const floatx4*>(scsrc + ((size_t)t * SB + sb) * 16);
+  };
+
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 acc[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[t][i] = zero;
+
+  const uint32_t slast = 4 * sb1 - 1;
+  u32x4 xr[XU], wr[3];  // the next step's x and the next weights on their way
+  float sx[4][2];
+  floatx4 xsc[4];
+  load_w(wr, 0, sb0);
+  load_x(xr, 4 * sb0);
+  put_w(0, wr, 0);
+  load_w(wr, 1, sb0);
+  put_w(0, wr, 1);
+  put_x(0, xr);
+  lds_barrier();
+  for (uint32_t sb = sb0; sb < sb1; ++sb) {
+    const uint32_t wcur = (sb - sb0) & 1;
+    const u32x4* wt = &wb[wcur][(wave * 32 + r) * 9];
+    floatx4 part[4][2], rest[4][2];
+    // Scales, one per byte (sub-blocks 0-3, 4-7), and 8*d*sc - dmin*mn of
+    // sub-blocks g and 4 + g.
+    uint32_t sc[2][2];
+    float d[2], mc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const u32x4 h = wt[16 * 9 * i];
+      sc[i][0] = h.y & 0x3F3F3F3Fu;
+      sc[i][1] = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+      const uint32_t mn0 = h.z & 0x3F3F3F3Fu;
+      const uint32_t mn1 = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
+      d[i] = half_bits_to_float(h.x);
+      const float dmin = half_bits_to_float(h.x >> 16);
+      const float d8 = 8.0f * d[i];
+      mc[i][0] = __builtin_fmaf(d8, (float)((sc[i][0] >> (8 * g)) & 0xFFu),
+                                -(dmin * (float)((mn0 >> (8 * g)) & 0xFFu)));
+      mc[i][1] = __builtin_fmaf(d8, (float)((sc[i][1] >> (8 * g)) & 0xFFu),
+                                -(dmin * (float)((mn1 >> (8 * g)) & 0xFFu)));
+    }
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      // Step s: its operands are in buffers it & 1.
+      const uint32_t s = 4 * sb + it;
+      const int b = it & 1;
+      load_x(xr, min(s + 1, slast));
+      if (it == 0) load_w(wr, 0, min(sb + 1, sb1 - 1));
+      if (it == 2) load_w(wr, 1, min(sb + 1, sb1 - 1));
+      if (it == 3) {
+        load_sx(sx, sb);
+        load_scale(xsc, sb);
+      }
+      u32x2 q[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        q[i] = reinterpret_cast<const u32x2*>(wt + 16 * 9 * i + 1 + 2 * it)[g];
+      // Weight tile i's operands for sub-block j.
+      auto weights = [&](f16x8 (&wq)[2], int j) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int k = 2 * it + j;
+          // sc as f16: the half 0x6400 | sc is 1024 + sc.
+          const uint32_t byte = (sc[i][k >> 2] >> (8 * (k & 3))) & 0xFFu;
+          const _Float16 sch = __builtin_bit_cast(_Float16, (unsigned short)(0x6400u | byte)) -
+                               (_Float16)1024.0f;
+          const u32x2 w = j ? q[i] : u32x2{q[i].x << 4, q[i].y << 4};
+          wq[i] = weights_f16(w, sch, sch * (_Float16)72.0f);
+        }
+      };
+      f16x8 xs[4][kParts], wq[2][2];
+      auto read_x = [&](int t, int j) {
+#pragma unroll
+        for (int c = 0; c < kParts; ++c)
+          xs[t][c] = __builtin_bit_cast(f16x8, xb[b][t][j][c][lane]);
+      };
+#pragma unroll
+      for (int t = 0; t < 4; ++t) read_x(t, 0);
+      weights(wq[0], 0);
+      weights(wq[1], 1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const bool first = it == 0 && j == 0;
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            part[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                xs[t][0], wq[j][i], first ? zero : part[t][i], 0, 0, 0);
+#pragma unroll
+          for (int c = 1; c < kParts; ++c)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              rest[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  xs[t][c], wq[j][i], first && c == 1 ? zero : rest[t][i], 0, 0, 0);
+          if (j == 0) read_x(t, 1);  // into the registers just used
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      // The other buffers were last read in step s - 1 (x) and in the
+      // super-block before (weights).
+      put_x(b ^ 1, xr);
+      if (it == 1) put_w(wcur ^ 1, wr, 0);
+      if (it == 3) put_w(wcur ^ 1, wr, 1);
+      lds_barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        floatx4 m = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[t][0], mc[i][0], zero, 0, 0, 0);
+        m = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[t][1], mc[i][1], m, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[t][i][e] += __builtin_fmaf(part[t][i][e] + rest[t][i][e], d[i] * xsc[t][e], m[e]);
+        pin(acc[t][i]);
+      }
+  }
+
+  float* y = p.y + z * p.y_split;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t mo = mb * kTileM + 16 * t + 4 * g + e;
+      if (mo >= p.M) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t no = nb * kTileN + wave * 32 + 16 * i + r;
+        if (no >= p.N) continue;
+        float v = acc[t][i][e];
+        if (p.ksplit == 1) {
+          if (!is_finite(v))
+            v = row_dot(p.w + (size_t)no * row_bytes, p.x + (size_t)mo * p.ldx, nullptr, p.K);
+          if (p.res) v += p.res[(size_t)mo * p.ldr + no];
+        }
+        y[(size_t)mo * p.ldy + no] = v;
+      }
+    }
+}
+
+// The K ranges' products added in range order, and the residual.
+__global__ __launch_bounds__(256) void q4k_tile_sum_kernel(const Q4kTileParams p,
+                                                           const float* __restrict__ part) {
+#pragma clang fp contract(off)
+  const uint32_t n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (n >= p.N) return;
+  const size_t i = (size_t)m * p.N + n;
+  float v = part[i];
+  for (uint32_t z = 1; z < p.ksplit; ++z) v += part[z * p.y_split + i];
+  if (!is_finite(v))
+    v = row_dot(p.w + (size_t)n * (p.K / kQ4kBlockWeights * kQ4kBlockBytes),
+                p.x + (size_t)m * p.ldx, nullptr, p.K);
+  if (p.res) v += p.res[(size_t)m * p.ldr + n];
+  p.y[(size_t)m * p.ldy + n] = v;
+}
+
 constexpr int kRowsWaves = 8;
 
 template <int NT, bool SWIGLU>
@@ -368,6 +739,69 @@ int launch_rows(const Q4kGemmParams& p, uint32_t ntiles, uint32_t mtiles, hipStr
   else
     hipLaunchKernelGGL((q4k_rows_kernel<NT, SWIGLU, false, kRowsWaves>), grid, block, 0, stream, p);
   STS_HIP(hipGetLastError());
+  return STS_OK;
+}
+
+// Many rows: x split once into the workspace, then the 64 x 128 tiles, in
+// chunks of at most kTileRows rows so that the workspace stays bounded.
+// *done stays false where the workspace is not to be had (the stream is being
+// captured and it would have to grow, or memory is short).
+constexpr uint32_t kTileRows = 1024;
+int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
+  const uint32_t KB = p.K / 32, SB = p.K / kQ4kBlockWeights;
+  const uint32_t nblocks = (p.N + kTileN - 1) / kTileN;
+  const uint32_t cus = (uint32_t)device_cu_count();
+  const uint32_t rows = (std::min(p.M, kTileRows) + kTileM - 1) / kTileM * kTileM;
+  // K ranges per output tile: as many as keep the launch within the two
+  // workgroups a CU holds, each at least four super-blocks.
+  const uint32_t tiles = nblocks * (rows / kTileM);
+  const uint32_t ksplit = std::max(1u, std::min(2 * cus / tiles, SB / 4));
+  const size_t plane_floats = TilePlanes::floats(rows, KB);
+  const size_t y_floats = ksplit > 1 ? (size_t)rows * p.N : 0;
+  Workspace* ws = nullptr;
+  if (int rc = try_workspace(stream, plane_floats + ksplit * y_floats, 0, &ws))
+    return rc;
+  if (!ws) return STS_OK;
+  const TilePlanes planes(ws->part, rows, KB);
+  float* part = ws->part + plane_floats;
+  for (uint32_t m0 = 0; m0 < p.M; m0 += kTileRows) {
+    Q4kTileParams t;
+    t.w = p.w[0];
+    t.units = planes.units;
+    t.sums = planes.sums;
+    t.scales = planes.scales;
+    t.x = p.x + (size_t)m0 * p.ldx;
+    t.res = p.res ? p.res + (size_t)m0 * p.ldr : nullptr;
+    t.y = p.y + (size_t)m0 * p.ldy;
+    t.ldx = p.ldx;
+    t.ldr = p.ldr;
+    t.ldy = p.ldy;
+    t.y_split = 0;
+    t.M = std::min(p.M - m0, kTileRows);
+    t.N = p.N;
+    t.K = p.K;
+    t.mtiles = (t.M + kTileM - 1) / kTileM;
+    t.ksplit = ksplit;
+    hipLaunchKernelGGL(split_planes_kernel, dim3((SB + 3) / 4, t.mtiles * 4), dim3(256), 0, stream,
+                       t.x, t.ldx, t.M, SB, planes.units, planes.sums, planes.scales);
+    STS_HIP(hipGetLastError());
+    const uint64_t grid = (uint64_t)((nblocks * ksplit + 7) / 8) * 8 * t.mtiles;
+    if (grid > 0x7FFFFFFFull) return fail(STS_ERR_INVALID, "GEMM N = %u too large", p.N);
+    Q4kTileParams k = t;
+    if (ksplit > 1) {
+      k.y = part;
+      k.ldy = p.N;
+      k.y_split = t.y_split = y_floats;
+    }
+    hipLaunchKernelGGL(q4k_tile_kernel, dim3((uint32_t)grid), dim3(256), 0, stream, k);
+    STS_HIP(hipGetLastError());
+    if (ksplit > 1) {
+      hipLaunchKernelGGL(q4k_tile_sum_kernel, dim3((p.N + 255) / 256, t.M), dim3(256), 0, stream,
+                         t, part);
+      STS_HIP(hipGetLastError());
+    }
+  }
+  *done = true;
   return STS_OK;
 }
 
@@ -404,6 +838,16 @@ int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   // against 19.2 us (13 x [12288, 4096]); and waves beyond eight leave too few
   // registers (12: 16.9 and 32.0 us).
   const uint64_t tiles = (uint64_t)ntiles * mtiles * p.Z;
+  // The tiles from 33 rows on, where the products outweigh their two extra
+  // launches (x split, K ranges summed): 48 rows x [12288, 4096] 37 against
+  // 50 us here, 112 x [4096, 4096] 33 against 51, but 80 x [4096, 4096] 32.5
+  // against 29.8, 32 x [12288, 4096] 34.6 against 29.7.
+  if (p.M > 32 && (uint64_t)mtiles * 16 * p.N * p.K >= 1500000000ull && p.Z == 1 && !p.swiglu_f &&
+      !p.norm_alpha) {
+    bool done = false;
+    if (int rc = launch_tiles(p, stream, &done)) return rc;
+    if (done) return STS_OK;
+  }
   if (p.swiglu_f) {
     if (tiles <= cus) return launch_rows<2, true>(p, ntiles, mtiles, stream);
     if (tiles <= 2 * cus) return launch_rows<4, true>(p, ntiles, mtiles, stream);

@@ -57,11 +57,77 @@ def test_rows_edges(gpu, M, N, K):
     check(host(sts_attn.q4k_gemm(dev(x), w)), blocks, x, N)
 
 
-@pytest.mark.parametrize("M,N,K", [(3, 40, 512), (20, 700, 1024)])
+# The tiles of many rows: 64 x 128 outputs, up to 1024 rows at a time, one or
+# several ranges of K.
+@pytest.mark.parametrize("M,N,K,res", [(33, 1921, 16384, True), (65, 4601, 4096, False),
+                                       (64, 11265, 2304, True), (130, 41001, 256, False),
+                                       (1025, 1501, 1024, True), (1088, 127, 11264, False)])
+def test_tiles_edges(gpu, M, N, K, res):
+    print(f"q4k tiles M={M} N={N} K={K} res={res}", flush=True)
+    blocks = oracle._random_q4k_scaled(M + N + K, N, K)
+    x = oracle.normal(N + 3 * M, (M, K))
+    x[M // 2, :K // 2] *= np.float32(1000.0)  # rows and super-blocks of other sizes
+    x[M - 1] *= np.float32(1e-12)
+    r = oracle.normal(N + 7, (M, N)) if res else None
+    w = sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))
+    got = host(sts_attn.q4k_gemm(dev(x), w, residual=dev(r) if res else None))
+    wt = torch.from_numpy(oracle.q4k_dequant(blocks, N, K)).cuda().double()
+    xd = dev(x).double()
+    ref = (xd @ wt.T.contiguous()).cpu().numpy() + (r.astype(np.float64) if res else 0.0)
+    tol = 1e-5 * q4k_bound(blocks, x, N) + (1e-6 * np.abs(r) if res else 0.0)
+    assert (np.abs(got - ref) <= tol).all(), (np.abs(got - ref) / tol).max()
+    again = host(sts_attn.q4k_gemm(dev(x), w, residual=dev(r) if res else None))
+    np.testing.assert_array_equal(again, got)
+
+
+def test_tiles_captured_without_workspace(gpu):
+    """A stream whose workspace does not hold the tiles' operands yet: captured,
+    the product runs without them; every replay gives the same values."""
+    M, N, K = 128, 4096, 4096
+    blocks = oracle._random_q4k_scaled(5, N, K)
+    x = oracle.normal(6, (M, K))
+    w = sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))
+    xd, out = dev(x), torch.empty((M, N), device="cuda")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        sts_attn.q4k_gemm(xd, w, out=out, stream=s)
+    ref = oracle.q4k_matvec_f64(blocks, x, N)
+    tol = 1e-5 * q4k_bound(blocks, x, N)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert (np.abs(host(out) - ref) <= tol).all()
+        eager = host(sts_attn.q4k_gemm(xd, w))
+        assert (np.abs(eager - ref) <= tol).all()
+
+
+@pytest.mark.parametrize("N,K,B,res", [(4096, 1024, 3, True), (4096, 1024, 4, True),
+                                       (300, 11264, 7, False), (300, 11264, 8, True),
+                                       (2048, 512, 70, False)])
+def test_matvec_batches(gpu, N, K, B, res):
+    """Rows of a batch on either side of the batch size from which they share
+    the weights: each within the bound of the f64 product."""
+    blocks = quantised(N + K, N, K)
+    x = oracle.normal(N + B, (B, K))
+    r = oracle.normal(N + 9, (B, N)) if res else None
+    w = sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))
+    got = host(sts_attn.q4k_matmul(dev(x[:, None]), w,
+                                   residual=dev(r[:, None]) if res else None))[:, 0]
+    check(got, blocks, x, N, r)
+
+
+# (40, 2400, 16384): the tiles of many rows, their K in several ranges;
+# (40, 41001, 1024): in one.
+@pytest.mark.parametrize("M,N,K", [(3, 40, 512), (20, 700, 1024), (40, 2400, 16384),
+                                   (40, 41001, 1024)])
 def test_rows_not_finite(gpu, M, N, K):
     """Row 0 holds an infinity, row 1 a NaN, row 2 values whose 15-fold
     overflows though the products do not; the others are ordinary."""
-    blocks = quantised(M * N + K, N, K)
+    blocks = (quantised if N * K < 1 << 20 else oracle._random_q4k_scaled)(M * N + K, N, K)
     wt = oracle.q4k_dequant(blocks, N, K).astype(np.float64)
     x = oracle.normal(N + M, (M, K))
     x[0, 37] = -np.inf
@@ -77,4 +143,5 @@ def test_rows_not_finite(gpu, M, N, K):
     big = x[2].astype(np.float64) @ wt.T
     np.testing.assert_allclose(got[2], big, rtol=1e-5, atol=1e-5 * np.abs(big).max())
     if M > 3:
-        check(got[3:], blocks, x[3:], N)
+        d = got[3:] - x[3:].astype(np.float64) @ wt.T
+        assert (np.abs(d) <= 1e-5 * q4k_bound(blocks, x[3:], N)).all()
