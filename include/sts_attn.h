@@ -413,7 +413,8 @@ int sts_debug_set_wait_limit(uint32_t polls);
  * n rows of k/256 super-blocks of 144 bytes.  x is [batch][k] (the
  * reference's [B, 1, K] input), y [batch][n], residual [batch][n] or NULL.
  * k must be a multiple of 256 and at most 16384; weights and x 16-byte
- * aligned.  Each batch row reads the whole weight matrix once.
+ * aligned.  From 4 rows on (8 where n < 2048) the rows share the weights as
+ * in sts_q4k_gemm, whose order of summation then applies.
  */
 int sts_q4k_matvec(const uint8_t* weights, const float* x, const float* residual, float* y,
                    uint32_t batch, uint32_t k, uint32_t n, void* stream);
