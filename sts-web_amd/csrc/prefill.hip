@@ -14,7 +14,7 @@
 //   is, after the online softmax, directly the B operand P^T of
 //   O^T = V^T P^T; the contraction order over keys is permuted identically
 //   in V^T and P^T, so P never goes through LDS.  Each tile's key range is
-//   also split over up to four workgroups (blockIdx.z); each publishes
+//   also split over up to eight workgroups (blockIdx.z); each publishes
 //   (O, max, sum) with device-coherent stores and the last to arrive folds
 //   them in split order.
 //
@@ -91,7 +91,7 @@ struct PrefillSmem {
   alignas(16) float vt[D * VP];
 };
 
-constexpr int kMaxPrefillSplits = 4;
+constexpr int kMaxPrefillSplits = 8;
 constexpr int kKsplit = 2;  // waves per query group (key slices of a block)
 
 // V^T is stored d-major with the 4-key quads of each row permuted by
@@ -526,6 +526,7 @@ __global__ __launch_bounds__(256 * KSPLIT) void prefill_kernel(const PrefillPara
 // consumer wave), so loading and converting overlap the matrix and softmax
 // work instead of alternating with it at workgroup barriers.
 constexpr int kWsStages = 4;
+constexpr uint32_t kMaxWsSplits = 16;
 constexpr int kWsKB = 64;
 // Lazy rescaling threshold of the bf16 kernels' online softmax (log2 units).
 constexpr float kLazyLog2 = 8.f;
@@ -625,7 +626,13 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
   const uint32_t base_w = p.len - p.S;
   const uint32_t q_last = min(p.S, (qt + 1) * QT) - 1;
   const uint32_t kend = min(p.len, base_w + q_last + 1);
-  const uint32_t nblk = (kend + KB - 1) / KB;
+  // This workgroup's share of the tile's key blocks: all of them, or with
+  // several splits (few tiles in the launch) blocks [blk0, blk0 + nblk).
+  const uint32_t nb_tile = (kend + KB - 1) / KB;
+  const uint32_t ns = min(p.nsplit, nb_tile), split = blockIdx.z;
+  if (split >= ns) return;  // the tile has fewer blocks than splits
+  const uint32_t blk0 = split * nb_tile / ns;
+  const uint32_t nblk = (split + 1) * nb_tile / ns - blk0;
   // Visit order of the key blocks: the tiles within two blocks of the
   // launch's longest take theirs last to first.  They then start on blocks
   // few other tiles read and end on the ones every tile of the head has
@@ -635,8 +642,8 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
   // keeps the forward order).  Step i of producers and consumers handles
   // block blk(i); steps past the last block stay past it (zero loads).
   const uint32_t maxblk = (p.len + KB - 1) / KB;
-  const bool reverse = !SPLIT && nblk + 2 >= maxblk;
-  auto blk = [&](uint32_t i) { return reverse && i < nblk ? nblk - 1 - i : i; };
+  const bool reverse = !SPLIT && p.nsplit == 1 && nblk + 2 >= maxblk;
+  auto blk = [&](uint32_t i) { return reverse && i < nblk ? nblk - 1 - i : blk0 + i; };
   if (tid < NS) {
     filled[tid] = 0;
     vfilled[tid] = 0;
@@ -1166,6 +1173,92 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
     dst[OT * 16 + 1] = lsum;
   }
   __syncthreads();
+  if (p.nsplit > 1) {
+    // Publish the split's unnormalised rows: per query group OT * 4 float4 and
+    // (max, sum) of every lane, whole kilobytes per store.
+    constexpr int RV = OT * 4;                     // float4 of a lane
+    constexpr int REC = 2 * 64 * (RV * 4 + 4);     // floats of a record
+    const size_t tile = (size_t)h * nqt + qt;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        coherent_rsrc(p.part + tile * p.nsplit * REC, ns * REC * sizeof(float));
+    // Byte offset of vector v (RV: the max and sum) of group gq in split s.
+    auto rec = [&](uint32_t s, int gq, int v) {
+      return (s * REC + ((gq * (RV + 1) + v) * 64 + lane) * 4) * (uint32_t)sizeof(float);
+    };
+    if (wave < 4 && ks == 0) {
+      const float* src = red + (qg * 64 + lane) * RS;
+      const float m2 = src[OT * 16], l2 = src[OT * 16 + 1];
+      const float mm = fmaxf(m, m2);
+      const float f1 = fast_exp2(m - mm), f2 = fast_exp2(m2 - mm);
+#pragma unroll
+      for (int v = 0; v < RV; ++v) {
+        coh_f4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o[v / 4][4 * (v % 4) + e] * f1 + src[4 * v + e] * f2;
+        st_coherent4(rsrc, rec(split, qg, v), y);
+      }
+      st_coherent4(rsrc, rec(split, qg, RV), coh_f4{mm, lsum * f1 + l2 * f2, 0.f, 0.f});
+      __builtin_amdgcn_s_waitcnt(0);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    __shared__ uint32_t s_ticket;
+    __syncthreads();
+    if (tid == 0) s_ticket = atomicAdd(p.counters + tile, 1u);
+    __syncthreads();
+    if (s_ticket != ns - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (tid == 0) atomicExch(p.counters + tile, 0u);
+    // Last to arrive: all eight waves fold the splits in split order, wave w
+    // the vectors RV/4 * (w / 2) .. of query group w % 2.
+    const int gq = wave & 1, v0 = RV / 4 * (wave >> 1);
+    const uint32_t qrow = qt * QT + gq * 32 + l32;
+    coh_f4 ml[kMaxWsSplits];
+#pragma unroll
+    for (int s = 0; s < kMaxWsSplits; ++s) {
+      ml[s] = coh_f4{-FLT_MAX, 0.f, 0.f, 0.f};
+      if (s < (int)ns) ml[s] = ld_coherent4(rsrc, rec(s, gq, RV));
+    }
+    coh_f4 y[RV / 4];
+    float mm = -FLT_MAX, l = 0.f;
+#pragma unroll
+    for (int v = 0; v < RV / 4; ++v) y[v] = coh_f4{0.f, 0.f, 0.f, 0.f};
+    constexpr int kAt = 8;  // splits in flight
+#pragma unroll
+    for (int s0 = 0; s0 < kMaxWsSplits; s0 += kAt) {
+      if (s0 >= (int)ns) break;
+      coh_f4 x[kAt][RV / 4];
+#pragma unroll
+      for (int s = 0; s < kAt; ++s)
+#pragma unroll
+        for (int v = 0; v < RV / 4; ++v) {
+          x[s][v] = coh_f4{0.f, 0.f, 0.f, 0.f};
+          if (s0 + s < (int)ns) x[s][v] = ld_coherent4(rsrc, rec(s0 + s, gq, v0 + v));
+        }
+      if (s0 == 0) {
+#pragma unroll
+        for (int s = 0; s < kMaxWsSplits; ++s) mm = fmaxf(mm, ml[s].x);
+      }
+#pragma unroll
+      for (int s = 0; s < kAt; ++s) {
+        const float f = fast_exp2(ml[s0 + s].x - mm);  // 0 past ns
+        l += f * ml[s0 + s].y;
+#pragma unroll
+        for (int v = 0; v < RV / 4; ++v)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[v][e] += f * x[s][v][e];
+      }
+    }
+    if (qrow >= p.S) return;
+    const float inv = 1.f / l;
+    float* orow = p.out + ((size_t)qrow * p.H + h) * D;
+#pragma unroll
+    for (int v = 0; v < RV / 4; ++v) {
+      const int t = (v0 + v) / 4, r = (v0 + v) % 4;
+      st4_stream(orow + 32 * t + 8 * r + 4 * hh,
+                 make_float4(y[v][0] * inv, y[v][1] * inv, y[v][2] * inv, y[v][3] * inv));
+    }
+    return;
+  }
   if (wave >= 4 || ks != 0 || !q_ok) return;
   const float* src = red + (qg * 64 + lane) * RS;
   const float m2 = src[OT * 16], l2 = src[OT * 16 + 1];
@@ -1186,6 +1279,32 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
     }
 }
 
+// Key-range splits of prefill_ws_kernel.  A launch with few tiles (short
+// chunks) leaves most CUs idle while each tile walks a long window alone, so
+// its blocks are dealt to as many workgroups as there are CUs, at least two
+// blocks each.  The splits' rows meet in memory (about 4 us), so the window
+// must shorten by six blocks or more for it (0.9 us a block).
+uint32_t ws_splits(uint32_t S, uint32_t H, uint32_t len) {
+  const uint32_t tiles = H * ((S + 63) / 64), nb = (len + kWsKB - 1) / kWsKB;
+  const uint32_t ns = std::min({(uint32_t)device_cu_count() / tiles, kMaxWsSplits, nb / 2});
+  return ns > 1 && nb - (nb + ns - 1) / ns >= 6 ? ns : 1u;
+}
+
+// The workspace of those splits; *nsplit falls back to 1 where it is not to be
+// had (the stream is being captured and it would have to grow).
+template <int D>
+int ws_workspace(uint32_t S, uint32_t H, uint32_t len, hipStream_t stream, uint32_t* nsplit,
+                 Workspace** out) {
+  *out = nullptr;
+  *nsplit = ws_splits(S, H, len);
+  if (*nsplit <= 1) return STS_OK;
+  const uint32_t tiles = H * ((S + 63) / 64);
+  if (int rc = try_workspace(stream, (size_t)tiles * *nsplit * 2 * 64 * (D / 2 + 4), tiles, out))
+    return rc;
+  if (!*out) *nsplit = 1;
+  return STS_OK;
+}
+
 template <int D, bool SPLIT, bool KV16 = false>
 int launch_ws(const PrefillParams& p, hipStream_t stream) {
   const uint32_t nqt = (p.S + 63) / 64;
@@ -1193,32 +1312,69 @@ int launch_ws(const PrefillParams& p, hipStream_t stream) {
   if ((uint64_t)p.M * D * sizeof(float) > 0x7FFFFFF0ull)
     return fail(STS_ERR_INVALID, "max_len %u too large for one head's buffer resource", p.M);
   PrefillParams q = p;
+  Workspace* ws = nullptr;
+  if (int rc = ws_workspace<D>(p.S, p.H, p.len, stream, &q.nsplit, &ws)) return rc;
+  if (ws) {
+    q.part = ws->part;
+    q.counters = ws->counters;
+  }
   // A sleeping workgroup costs nothing only while no other waits for its CU.
-  q.start_stagger = KV16 && !SPLIT && (uint64_t)p.H * nqt <= (uint64_t)device_cu_count() ? 10u : 0u;
-  hipLaunchKernelGGL((prefill_ws_kernel<D, SPLIT, KV16>), dim3(p.H, nqt, 1), dim3(512), 0, stream,
-                     q);
+  q.start_stagger = KV16 && !SPLIT && q.nsplit == 1 &&
+                            (uint64_t)p.H * nqt <= (uint64_t)device_cu_count()
+                        ? 10u
+                        : 0u;
+  hipLaunchKernelGGL((prefill_ws_kernel<D, SPLIT, KV16>), dim3(p.H, nqt, q.nsplit), dim3(512), 0,
+                     stream, q);
   STS_HIP(hipGetLastError());
   return STS_OK;
 }
 
-// Key-range splits of the f32 kernel: f32 tiles carry four times the MFMA
-// work of bf16 ones, so their key ranges are split until there are about two
-// workgroups per CU.
-uint32_t f32_splits(uint32_t S, uint32_t H) {
-  const uint32_t tiles = H * ((S + kBQ - 1) / kBQ);
-  const uint32_t cus = (uint32_t)device_cu_count();
-  const uint32_t nsplit = (2 * cus + tiles - 1) / tiles;
-  return std::max(1u, std::min<uint32_t>(nsplit, kMaxPrefillSplits));
+// Key-range splits of the f32 kernel.  Its workgroups run one per CU, so a
+// launch takes rounds of them; the cost of ns splits in units of one key block
+// (about 4.8 us) is the larger of the longest workgroup and the rounds at the
+// average tile, a block's worth of start and merge per workgroup and a little
+// for each record of the fold.  24 queries after 2500 cached: 8 splits 36.7 us
+// (4: 56.8); 300 after 1100: 3 splits 84 (4: 92); 130 after 2500: 5 splits 98
+// (4: 111); 512 after 256: 2 splits 55.9 (3: 60.9).
+uint32_t f32_splits(uint32_t S, uint32_t H, uint32_t len) {
+  const uint32_t tiles = H * ((S + kBQ - 1) / kBQ), cus = (uint32_t)device_cu_count();
+  const uint32_t longest = (len + kBK - 1) / kBK;
+  const uint32_t shortest = (len - S + std::min<uint32_t>(S, kBQ) + kBK - 1) / kBK;
+  const float average = 0.5f * (float)(longest + shortest);
+  uint32_t best = 1;
+  float least = FLT_MAX;
+  for (uint32_t ns = 1; ns <= std::min<uint32_t>(kMaxPrefillSplits, longest); ++ns) {
+    const float rounds = (float)(((uint64_t)tiles * ns + cus - 1) / cus);
+    const float cost = std::max((float)longest / ns + 1.f, rounds * (average / ns + 1.f)) + 0.25f * ns;
+    if (cost < least) {
+      least = cost;
+      best = ns;
+    }
+  }
+  return best;
 }
 
-// The split workspace of the f32 kernel (null with one split).
+// The split workspace of the f32 kernel (null with one split).  Also where
+// fewer are wanted it is made large enough for about two workgroups per CU, up
+// to four splits a tile, whatever the window: a call captured later with a
+// longer window finds at least that many and makes do with them.
 template <int D>
-int f32_workspace(uint32_t S, uint32_t H, hipStream_t stream, uint32_t* nsplit, Workspace** out) {
+int f32_workspace(uint32_t S, uint32_t H, uint32_t len, hipStream_t stream, uint32_t* nsplit,
+                  Workspace** out) {
   *out = nullptr;
-  *nsplit = f32_splits(S, H);
-  if (*nsplit <= 1) return STS_OK;
   const uint32_t tiles = H * ((S + kBQ - 1) / kBQ);
-  return get_workspace(stream, (size_t)tiles * *nsplit * 256 * (D / 4 + 2), tiles, out);
+  const uint32_t cus = (uint32_t)device_cu_count();
+  const uint32_t base = std::min((2 * cus + tiles - 1) / tiles, 4u);
+  const size_t rec = 256 * (D / 4 + 2);
+  *nsplit = f32_splits(S, H, len);
+  const uint32_t most = std::max(base, *nsplit);
+  if (most <= 1) return STS_OK;
+  if (int rc = try_workspace(stream, (size_t)tiles * most * rec, tiles, out)) return rc;
+  if (!*out) {
+    *nsplit = base;
+    if (base > 1) return get_workspace(stream, (size_t)tiles * base * rec, tiles, out);
+  }
+  return STS_OK;
 }
 
 template <int D>
@@ -1229,7 +1385,7 @@ int launch_f32(const PrefillParams& p, hipStream_t stream) {
     return fail(STS_ERR_INVALID, "max_len %u too large for one head's buffer resource", p.M);
   PrefillParams q = p;
   Workspace* ws = nullptr;
-  if (int rc = f32_workspace<D>(p.S, p.H, stream, &q.nsplit, &ws)) return rc;
+  if (int rc = f32_workspace<D>(p.S, p.H, p.len, stream, &q.nsplit, &ws)) return rc;
   if (ws) {
     q.part = ws->part;
     q.counters = ws->counters;
@@ -1301,11 +1457,13 @@ int reserve_prefill(uint32_t S, uint32_t H, uint32_t len, uint32_t head_dim, int
   if (int rc = device_error_word(&err)) return rc;
   if (head_dim != 64 && head_dim != 128)
     return reserve_decode(S, H, head_dim, len, stream);  // launch_prefill_by_decode's plan
-  if (bf16_rows || precision != STS_PREC_F32) return STS_OK;  // no workspace
   uint32_t nsplit = 1;
   Workspace* ws = nullptr;
-  return head_dim == 128 ? f32_workspace<128>(S, H, stream, &nsplit, &ws)
-                         : f32_workspace<64>(S, H, stream, &nsplit, &ws);
+  if (bf16_rows || precision != STS_PREC_F32)
+    return head_dim == 128 ? ws_workspace<128>(S, H, len, stream, &nsplit, &ws)
+                           : ws_workspace<64>(S, H, len, stream, &nsplit, &ws);
+  return head_dim == 128 ? f32_workspace<128>(S, H, len, stream, &nsplit, &ws)
+                         : f32_workspace<64>(S, H, len, stream, &nsplit, &ws);
 }
 
 int launch_prefill(const PrefillParams& p0, uint32_t head_dim, int precision, hipStream_t stream) {
