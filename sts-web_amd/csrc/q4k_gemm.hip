@@ -358,6 +358,164 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
   }
 }
 
+// One weight of a slot after the other is what a single row of x is worth: no
+// 16-row tile to fill.  The 64 weights of slot s of a row (iteration s % 4 of
+// super-block s / 4) against the lane's x values: the nibble in a byte's upper
+// half with its top bit flipped is 16 (q - 8) as a signed byte, so no offset has
+// to cancel (the min takes 8 d sc off again).
+__device__ __forceinline__ float slot_dot8(u32x4 hd, u32x4 qa, u32x4 qb, uint32_t j,
+                                           const float (&x)[64], float sl, float sh) {
+  const float d = half_bits_to_float(hd.x), dmin = half_bits_to_float(hd.x >> 16);
+  uint32_t scl, mnl, sch, mnh;
+  scale_min(hd.y, hd.z, hd.w, j, scl, mnl);
+  scale_min(hd.y, hd.z, hd.w, j + 1, sch, mnh);
+  const uint32_t words[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+  float ql[4] = {0.f, 0.f, 0.f, 0.f}, qh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    const uint32_t lo = ((words[w] << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
+    const uint32_t hi = (words[w] & 0xF0F0F0F0u) ^ 0x80808080u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ql[i] = __builtin_fmaf((float)(int8_t)(lo >> (8 * i)), x[4 * w + i], ql[i]);
+      qh[i] = __builtin_fmaf((float)(int8_t)(hi >> (8 * i)), x[32 + 4 * w + i], qh[i]);
+    }
+  }
+  const float d1 = d * (float)scl * 0.0625f, d2 = d * (float)sch * 0.0625f;  // exact
+  const float m1 = __builtin_fmaf(128.f, d1, -(dmin * (float)mnl));
+  const float m2 = __builtin_fmaf(128.f, d2, -(dmin * (float)mnh));
+  const float a = __builtin_fmaf(d1, (ql[0] + ql[1]) + (ql[2] + ql[3]), m1 * sl);
+  const float b = __builtin_fmaf(d2, (qh[0] + qh[1]) + (qh[2] + qh[3]), m2 * sh);
+  return a + b;
+}
+
+// q4k_vec_kernel: one or two rows of x (the depformer of one conversation),
+// where the products are a few microseconds of latency.  One wave per
+// workgroup takes RPW weight rows at once, a slot per lane (64 / RPW lanes a
+// row), R times; it stages its row of x in LDS by itself, so no barrier stands
+// in its way, and with NORM sums its squares on the way.  1 row: [3072, 1024]
+// with RMSNorm 4.0 us against 5.8 in q4k_rows_kernel, [5632, 1024] with SwiGLU
+// 4.9 against 6.9, [1024, 2816] 4.0 against about 7; [1024, 1024] 3.5, of which
+// an empty launch is 2.5.  XL: float4 of x per lane, K <= 256 XL.
+template <int XL, int R, bool NORM, bool SWIGLU>
+__global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
+#pragma clang fp contract(off)
+  constexpr int RPW = XL <= 4 ? 4 : XL <= 8 ? 2 : 1;
+  constexpr int LPR = 64 / RPW;  // lanes of a row
+  constexpr int NH = SWIGLU ? 2 : 1;
+  __shared__ __align__(16) float xs[XL * 4][68];  // slot, its 64 values (pitch 68)
+  const int lane = threadIdx.x;
+  const int s = lane % LPR;
+  const uint32_t b = blockIdx.y, z = blockIdx.z;
+  const uint8_t* W = p.w[z];
+  const float* X = p.x + z * p.x_zstride + (size_t)b * p.ldx;
+  const uint32_t nout = SWIGLU ? p.swiglu_f : p.N;
+  const size_t row_bytes = (size_t)(p.K / kQ4kBlockWeights) * kQ4kBlockBytes;
+  // A lane past the row's last slot reads slot 0 with its d and dmin as zeros.
+  const bool has = (uint32_t)s < p.K / 64;
+  const uint32_t slot = has ? s : 0u;
+  const uint32_t row0 = blockIdx.x * (R * RPW) + lane / LPR;
+
+  // x (and alpha) first, then the weights and the residual.
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(X), 0, (int)(p.K * sizeof(float)), kGemmBufferWord3);
+  const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(p.norm_alpha), 0, (int)(p.K * sizeof(float)), kGemmBufferWord3);
+  float4 xr[XL], al[NORM ? XL : 1];
+#pragma unroll
+  for (int k = 0; k < XL; ++k) {
+    const uint32_t o = (lane + 64 * k) * 16;  // past K: zeros
+    xr[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, o, 0, 0));
+    if constexpr (NORM)
+      al[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ars, o, 0, 0));
+  }
+  u32x4 hd[R][NH], qa[R][NH], qb[R][NH];
+  float res[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const uint32_t n = min(row0 + j * RPW, nout - 1);
+#pragma unroll
+    for (int hv = 0; hv < NH; ++hv) {
+      const uint8_t* blk = W + (n + (hv ? p.swiglu_f : 0u)) * row_bytes +
+                           (size_t)(slot >> 2) * kQ4kBlockBytes;
+      hd[j][hv] = ld16(blk);
+      hd[j][hv].x = has ? hd[j][hv].x : 0u;
+      qa[j][hv] = ld16(blk + 16 + 32 * (slot & 3u));
+      qb[j][hv] = ld16(blk + 32 + 32 * (slot & 3u));
+    }
+    res[j] = p.res ? p.res[(size_t)b * p.ldr + n] : 0.f;
+  }
+  float ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < XL; ++k) {
+    float4 v = xr[k];
+    if constexpr (NORM) {
+      ss[0] = __builtin_fmaf(v.x, v.x, ss[0]);
+      ss[1] = __builtin_fmaf(v.y, v.y, ss[1]);
+      ss[2] = __builtin_fmaf(v.z, v.z, ss[2]);
+      ss[3] = __builtin_fmaf(v.w, v.w, ss[3]);
+      v = make_float4(v.x * al[k].x, v.y * al[k].y, v.z * al[k].z, v.w * al[k].w);
+    }
+    const int i = lane + 64 * k;
+    *reinterpret_cast<float4*>(&xs[i >> 4][4 * (i & 15)]) = v;
+  }
+  __syncthreads();  // one wave: orders its LDS writes before its reads
+  float x[64];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float4 t = *reinterpret_cast<const float4*>(&xs[slot][4 * j]);
+    x[4 * j] = t.x;
+    x[4 * j + 1] = t.y;
+    x[4 * j + 2] = t.z;
+    x[4 * j + 3] = t.w;
+  }
+  float sl[4] = {0.f, 0.f, 0.f, 0.f}, sh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    sl[j & 3] += x[j];
+    sh[j & 3] += x[32 + j];
+  }
+  const float sxl = (sl[0] + sl[1]) + (sl[2] + sl[3]), sxh = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  auto lanes_sum = [&](float v) {
+    v += xchg<0>(v);
+    v += xchg<1>(v);
+    v += xchg<2>(v);
+    v += xchg<3>(v);
+    if constexpr (LPR >= 32) v = sum_xor16(v);
+    if constexpr (LPR >= 64) v = sum_xor32(v);
+    return v;
+  };
+  float inv = 1.f;
+  if constexpr (NORM) {
+    float q = (ss[0] + ss[1]) + (ss[2] + ss[3]);
+    q += xchg<0>(q);
+    q += xchg<1>(q);
+    q += xchg<2>(q);
+    q += xchg<3>(q);
+    q = sum_xor32(sum_xor16(q));
+    inv = 1.0f / sqrtf(q / (float)p.K + p.norm_eps);
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const uint32_t n = row0 + j * RPW;
+    float v[NH];
+#pragma unroll
+    for (int hv = 0; hv < NH; ++hv)
+      v[hv] = lanes_sum(slot_dot8(hd[j][hv], qa[j][hv], qb[j][hv], 2 * (slot & 3u), x, sxl, sxh));
+    if (s != 0 || n >= nout) continue;
+#pragma unroll
+    for (int hv = 0; hv < NH; ++hv) {
+      if (!is_finite(v[hv]))
+        v[hv] = row_dot(W + (n + (hv ? p.swiglu_f : 0u)) * row_bytes, X, p.norm_alpha, p.K);
+      v[hv] *= inv;
+    }
+    float o = v[0];
+    if constexpr (SWIGLU) o = o / (1.0f + expf(-o)) * v[NH - 1];
+    if (p.res) o += res[j];
+    p.y[z * p.y_zstride + (size_t)b * p.ldy + n] = o;
+  }
+}
+
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -742,6 +900,19 @@ int launch_rows(const Q4kGemmParams& p, uint32_t ntiles, uint32_t mtiles, hipStr
   return STS_OK;
 }
 
+template <int XL, int R>
+int launch_vec(const Q4kGemmParams& p, uint32_t nout, hipStream_t stream) {
+  constexpr uint32_t rows = R * (XL <= 4 ? 4 : XL <= 8 ? 2 : 1);
+  const dim3 grid((nout + rows - 1) / rows, p.M, p.Z), block(64);
+  auto kernel = p.swiglu_f ? (p.norm_alpha ? q4k_vec_kernel<XL, R, true, true>
+                                           : q4k_vec_kernel<XL, R, false, true>)
+                           : (p.norm_alpha ? q4k_vec_kernel<XL, R, true, false>
+                                           : q4k_vec_kernel<XL, R, false, false>);
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, p);
+  STS_HIP(hipGetLastError());
+  return STS_OK;
+}
+
 // Many rows: x split once into the workspace, then the 64 x 128 tiles, in
 // chunks of at most kTileRows rows so that the workspace stays bounded.
 // *done stays false where the workspace is not to be had (the stream is being
@@ -831,6 +1002,21 @@ int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   const uint32_t nout = p.swiglu_f ? p.swiglu_f : p.N;
   const uint32_t ntiles = (nout + 15) / 16;
   const uint32_t cus = (uint32_t)device_cu_count();
+  // One or two rows of x, measured against q4k_rows_kernel: 1 x [48000, 1024]
+  // 9.4 and 16.7 us, [48000, 4096] 33.3 and 47.1; 2 x [48000, 1024] 14.6 and
+  // 16.8, [48000, 2048] 28.9 and 29.1, [4096, 4096] 7.7 and 9.2.  The second row
+  // unpacks the weights again, which beyond that costs more than the 16-row
+  // tile: 2 x [16384, 3072] 20.5 and 14.1, [48000, 4096] 57.9 and 47.4.
+  if (p.K <= 4096 && (p.M == 1 || (p.M == 2 && (p.K <= 2048 || nout * p.Z <= 16 * cus)))) {
+    // A wave per few weight rows; where that would be more than eight waves a
+    // CU, four times the rows.
+    const uint64_t waves = (uint64_t)nout * p.M * p.Z / (p.K <= 1024 ? 4 : p.K <= 2048 ? 2 : 1);
+    const bool many = waves > 8ull * cus;
+    if (p.K <= 1024) return many ? launch_vec<4, 4>(p, nout, stream) : launch_vec<4, 1>(p, nout, stream);
+    if (p.K <= 2048) return many ? launch_vec<8, 4>(p, nout, stream) : launch_vec<8, 1>(p, nout, stream);
+    if (p.K <= 3072) return many ? launch_vec<12, 4>(p, nout, stream) : launch_vec<12, 1>(p, nout, stream);
+    return many ? launch_vec<16, 4>(p, nout, stream) : launch_vec<16, 1>(p, nout, stream);
+  }
   // Weight tiles per workgroup: as many as bring the launch to about one
   // workgroup per CU, up to six (eight spill registers).  Every workgroup splits
   // its x rows itself, so fewer and larger workgroups split them less often:

@@ -57,6 +57,62 @@ def test_rows_edges(gpu, M, N, K):
     check(host(sts_attn.q4k_gemm(dev(x), w)), blocks, x, N)
 
 
+# One or two rows: a weight row per 16, 32 or 64 lanes (K up to 1024, 2048,
+# 4096), one or four of them a wave; with and without RMSNorm, SwiGLU, residual.
+@pytest.mark.parametrize("M,N,K,norm,swiglu,res", [
+    (1, 1, 256, False, False, False), (2, 30, 768, True, True, False),
+    (1, 3073, 1024, True, False, True), (2, 9001, 1024, False, False, True),
+    (1, 20002, 512, True, True, False), (1, 66, 1280, False, True, False),
+    (2, 6003, 2048, True, False, False), (1, 1024, 2816, False, False, True),
+    (2, 5001, 3072, True, False, True), (1, 2817, 4096, True, False, False),
+    (2, 1500, 3328, False, True, False), (1, 515, 4352, False, False, True),
+    (2, 4096, 2304, True, False, False), (2, 4097, 2304, True, False, False)])
+def test_single_rows(gpu, M, N, K, norm, swiglu, res):
+    print(f"q4k M={M} N={N} K={K} norm={norm} swiglu={swiglu} res={res}", flush=True)
+    blocks = oracle._random_q4k_scaled(M + N + K, N, K)
+    x = oracle.normal(N + M, (M, K)) * np.float32(2.0)
+    alpha = (1 + 0.1 * oracle.normal(K, (K,))).astype(np.float32)
+    r = oracle.normal(N + 3, (M, N)) if res else None
+    w = sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))
+    got = host(sts_attn.q4k_gemm(dev(x), w, residual=dev(r) if res else None, swiglu=swiglu,
+                                 norm_alpha=dev(alpha) if norm else None, norm_eps=1e-8))
+    xn = oracle.rmsnorm_wgsl(x, alpha, 1e-8) if norm else x
+    y = oracle.q4k_matvec_f64(blocks, xn, N)
+    b = 1e-5 * q4k_bound(blocks, xn, N)
+    if swiglu:
+        F = N // 2
+        g, v = y[:, :F], y[:, F:]
+        sig = 1 / (1 + np.exp(-g))
+        want = g * sig * v
+        tol = (np.abs(sig * (1 + g * (1 - sig))) * np.abs(v) * b[:, :F]
+               + np.abs(g * sig) * b[:, F:] + 1e-6 * np.abs(want) + 1e-30)
+    else:
+        want, tol = y, b
+    if res:
+        want, tol = want + r, tol + 1e-6 * np.abs(r)
+    d = got.astype(np.float64) - want
+    assert (np.abs(d) <= tol).all(), (np.abs(d) / tol).max()
+    if not norm and not swiglu:
+        assert np.linalg.norm(d) <= 3e-7 * np.linalg.norm(want)
+
+
+def test_single_rows_not_finite(gpu):
+    N, K = 300, 1024
+    blocks = oracle._random_q4k_scaled(8, N, K)
+    wt = oracle.q4k_dequant(blocks, N, K).astype(np.float64)
+    w = sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))
+    x = oracle.normal(9, (2, K))
+    x[0, 37] = np.inf
+    x[1] = 0
+    x[1, 5], x[1, K - 2] = np.float32(3e38), np.float32(-1e38)
+    got = host(sts_attn.q4k_gemm(dev(x), w))
+    with np.errstate(invalid="ignore"):
+        want = np.where(wt[:, 37] == 0, np.nan, np.inf * np.sign(wt[:, 37]))
+    np.testing.assert_array_equal(got[0], want.astype(np.float32))
+    big = x[1].astype(np.float64) @ wt.T
+    np.testing.assert_allclose(got[1], big, rtol=1e-5, atol=1e-5 * np.abs(big).max())
+
+
 # The tiles of many rows: 64 x 128 outputs, up to 1024 rows at a time, one or
 # several ranges of K.
 @pytest.mark.parametrize("M,N,K,res", [(33, 1921, 16384, True), (65, 4601, 4096, False),
