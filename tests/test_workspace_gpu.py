@@ -217,3 +217,40 @@ def test_device_errors_refused_inside_capture(gpu, fresh_stream):
     s.synchronize()
     assert torch.equal(x, torch.full((16,), 2.0, device="cuda"))
     assert sts_attn.device_errors(stream=s) == 0
+
+
+@pytest.mark.parametrize("where", ["default", "side", "nested", "thread", "capture"])
+def test_current_stream_handle(gpu, where):
+    """A call without a stream goes to the calling thread's current one."""
+    import threading
+    import torch
+
+    def same():
+        return sts_attn._stream(None) == torch.cuda.current_stream().cuda_stream
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    if where == "default":
+        assert same()
+    elif where in ("side", "nested"):
+        with torch.cuda.stream(a):
+            assert same() and sts_attn._stream(None) == a.cuda_stream
+            if where == "nested":
+                with torch.cuda.stream(b):
+                    assert sts_attn._stream(None) == b.cuda_stream
+                assert sts_attn._stream(None) == a.cuda_stream
+    elif where == "thread":
+        got = []
+        with torch.cuda.stream(a):  # current in this thread only
+            t = threading.Thread(target=lambda: got.append((sts_attn._stream(None), same())))
+            t.start()
+            t.join()
+        assert got == [(torch.cuda.default_stream().cuda_stream, True)]
+    else:
+        x, y = torch.zeros(4, device="cuda"), torch.zeros(4, device="cuda")
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            assert same()
+            y.copy_(x)
+        g.replay()
+        torch.cuda.synchronize()
+    assert sts_attn._stream(a) == a.cuda_stream and sts_attn._stream(7) == 7
