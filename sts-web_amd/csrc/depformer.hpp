@@ -36,6 +36,23 @@ struct Q4kGemmParams {
 // K above 4096 takes no RMSNorm or SwiGLU and Z = 1 only.  (q4k_gemm.hip)
 int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream);
 
+// One decode step's attention (heads of 64) and its output projection in one
+// launch, M <= 2 rows, K <= 1024: p.x is not read, x is the attention of row
+// b's q over slots 0..len-1 of its cache [K/64][max_len][64], slot len-1 being
+// k_new / v_new, which the launch also writes to the cache.  scale_log2 =
+// scale * log2(e).
+struct DepthAttention {
+  const float* q = nullptr;
+  const float* k_new = nullptr;
+  const float* v_new = nullptr;
+  float* k = nullptr;
+  float* v = nullptr;
+  uint64_t q_bstride = 0, kv_bstride = 0;  // floats
+  uint32_t len = 0, max_len = 0;
+  float scale_log2 = 0.f;
+};
+int launch_q4k_attention(const Q4kGemmParams& p, const DepthAttention& a, hipStream_t stream);
+
 // out[b][i] = x[b][i] * (1 / sqrt(sum x^2 / D + eps)) * alpha[i] in the
 // order of shader_rmsnorm.wgsl:27-92, one workgroup per row.
 int launch_rmsnorm(const float* x, const float* alpha, float* out, uint32_t rows, uint32_t D,

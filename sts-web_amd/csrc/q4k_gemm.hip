@@ -23,6 +23,7 @@
 // plain product has them.
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "common.hpp"
 #include "depformer.hpp"
@@ -389,6 +390,118 @@ __device__ __forceinline__ float slot_dot8(u32x4 hd, u32x4 qa, u32x4 qb, uint32_
   return a + b;
 }
 
+// Decode attention of all heads (dim 64) of one stream over the slots 0..len-1
+// of its cache in one wave, slot len-1 being k_new / v_new: head 4k + lane/16
+// in registers k, dims 4c..4c+3 with c = lane % 16.  Four slots at a time,
+// online softmax, as decode_kernel has it.  Buffer loads past a resource (a
+// head or slot that is not there) give zeros.
+template <int NK>
+struct SlotAttention {
+  float4 q[NK], kn[NK], vn[NK], kk[4][NK], vv[4][NK];
+  __amdgpu_buffer_rsrc_t krs, vrs;
+  uint32_t off[NK];  // of slot 0 of the head in the cache, or kSkip
+  int lane;
+
+  static __device__ __forceinline__ float4 ld(__amdgpu_buffer_rsrc_t rs, uint32_t o) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0));
+  }
+  __device__ __forceinline__ void load(const DepthAttention& a, uint32_t t0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const uint32_t o = t0 + j < a.len - 1 && off[k] != kSkip ? off[k] + (t0 + j) * 256 : kSkip;
+        kk[j][k] = ld(krs, o);
+        vv[j][k] = ld(vrs, o);
+      }
+  }
+  __device__ __forceinline__ void begin(const DepthAttention& a, uint32_t b, uint32_t dim, int l) {
+    lane = l;
+    const uint32_t row = dim * (uint32_t)sizeof(float), head = a.max_len * 256;
+    auto row_of = [&](const float* p) {
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p) + b * a.q_bstride, 0,
+                                               (int)row, kGemmBufferWord3);
+    };
+    const __amdgpu_buffer_rsrc_t qrs = row_of(a.q), knrs = row_of(a.k_new), vnrs = row_of(a.v_new);
+    const int cache = (int)(dim / 64 * head);
+    krs = __builtin_amdgcn_make_buffer_rsrc(a.k + b * a.kv_bstride, 0, cache, kGemmBufferWord3);
+    vrs = __builtin_amdgcn_make_buffer_rsrc(a.v + b * a.kv_bstride, 0, cache, kGemmBufferWord3);
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      const uint32_t h = 4 * k + lane / 16;
+      off[k] = h < dim / 64 ? h * head + (lane & 15) * 16 : kSkip;
+      q[k] = ld(qrs, (lane + 64 * k) * 16);
+      kn[k] = ld(knrs, (lane + 64 * k) * 16);
+      vn[k] = ld(vnrs, (lane + 64 * k) * 16);
+    }
+    load(a, 0);
+  }
+  __device__ __forceinline__ void store_new(const DepthAttention& a, uint32_t b) {
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      if (off[k] == kSkip) continue;
+      const size_t o = b * a.kv_bstride + off[k] / 4 + (a.len - 1) * 64;
+      *reinterpret_cast<float4*>(a.k + o) = kn[k];
+      *reinterpret_cast<float4*>(a.v + o) = vn[k];
+    }
+  }
+  __device__ __forceinline__ void finish(const DepthAttention& a, float4 (&out)[NK]) {
+    float m[NK], l[NK];
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      m[k] = -3.402823466e+38f;
+      l[k] = 0.f;
+      out[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+      q[k] = make_float4(q[k].x * a.scale_log2, q[k].y * a.scale_log2, q[k].z * a.scale_log2,
+                         q[k].w * a.scale_log2);
+    }
+    for (uint32_t t0 = 0; t0 < a.len; t0 += 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (t0 + j != a.len - 1) continue;
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+          kk[j][k] = kn[k];
+          vv[j][k] = vn[k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        float s[4], mn = m[k];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float4 t = kk[j][k];
+          float d = __builtin_fmaf(q[k].w, t.w, __builtin_fmaf(q[k].z, t.z,
+                    __builtin_fmaf(q[k].y, t.y, q[k].x * t.x)));
+          d += xchg<0>(d);
+          d += xchg<1>(d);
+          d += xchg<2>(d);
+          d += xchg<3>(d);
+          s[j] = t0 + j < a.len ? d : -INFINITY;
+          mn = fmaxf(mn, s[j]);
+        }
+        const float al = __builtin_amdgcn_exp2f(m[k] - mn);
+        m[k] = mn;
+        l[k] *= al;
+        out[k] = make_float4(out[k].x * al, out[k].y * al, out[k].z * al, out[k].w * al);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float w = __builtin_amdgcn_exp2f(s[j] - mn);
+          l[k] += w;
+          out[k].x = __builtin_fmaf(w, vv[j][k].x, out[k].x);
+          out[k].y = __builtin_fmaf(w, vv[j][k].y, out[k].y);
+          out[k].z = __builtin_fmaf(w, vv[j][k].z, out[k].z);
+          out[k].w = __builtin_fmaf(w, vv[j][k].w, out[k].w);
+        }
+      }
+      if (t0 + 4 < a.len) load(a, t0 + 4);
+    }
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+      out[k] = make_float4(out[k].x / l[k], out[k].y / l[k], out[k].z / l[k], out[k].w / l[k]);
+  }
+};
+
 // q4k_vec_kernel: one or two rows of x (the depformer of one conversation),
 // where the products are a few microseconds of latency.  One wave per
 // workgroup takes RPW weight rows at once, a slot per lane (64 / RPW lanes a
@@ -397,13 +510,23 @@ __device__ __forceinline__ float slot_dot8(u32x4 hd, u32x4 qa, u32x4 qb, uint32_
 // with RMSNorm 4.0 us against 5.8 in q4k_rows_kernel, [5632, 1024] with SwiGLU
 // 4.9 against 6.9, [1024, 2816] 4.0 against about 7; [1024, 1024] 3.5, of which
 // an empty launch is 2.5.  XL: float4 of x per lane, K <= 256 XL.
-template <int XL, int R, bool NORM, bool SWIGLU>
-__global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
+//
+// ATTN: x is the output of one decode step's attention over a few slots, which
+// every wave computes for itself from q, k_new, v_new and the cache (XL float4
+// a lane: head 4k + lane / 16, 16 lanes a row); the first workgroup of a row
+// writes the new slot, which the others take from k_new and v_new.
+// [1024, 1024], 16 heads: 4.6 us to four slots, 5.8 to eight, where the two
+// launches were 7.0; the second four slots are a second round trip to memory.
+struct NoAttention {};
+template <int XL, int R, bool NORM, bool SWIGLU, typename A = NoAttention>
+__global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p, const A a) {
 #pragma clang fp contract(off)
+  constexpr bool ATTN = !std::is_same_v<A, NoAttention>;
   constexpr int RPW = XL <= 4 ? 4 : XL <= 8 ? 2 : 1;
   constexpr int LPR = 64 / RPW;  // lanes of a row
   constexpr int NH = SWIGLU ? 2 : 1;
   __shared__ __align__(16) float xs[XL * 4][68];  // slot, its 64 values (pitch 68)
+  __shared__ __align__(16) float xc[ATTN ? XL * 256 : 4];  // for row_dot
   const int lane = threadIdx.x;
   const int s = lane % LPR;
   const uint32_t b = blockIdx.y, z = blockIdx.z;
@@ -422,8 +545,10 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(p.norm_alpha), 0, (int)(p.K * sizeof(float)), kGemmBufferWord3);
   float4 xr[XL], al[NORM ? XL : 1];
+  SlotAttention<ATTN ? XL : 1> at;
+  if constexpr (ATTN) at.begin(a, b, p.K, lane);
 #pragma unroll
-  for (int k = 0; k < XL; ++k) {
+  for (int k = 0; k < (ATTN ? 0 : XL); ++k) {
     const uint32_t o = (lane + 64 * k) * 16;  // past K: zeros
     xr[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, o, 0, 0));
     if constexpr (NORM)
@@ -445,6 +570,10 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
     }
     res[j] = p.res ? p.res[(size_t)b * p.ldr + n] : 0.f;
   }
+  if constexpr (ATTN) {
+    if (blockIdx.x == 0) at.store_new(a, b);
+    at.finish(a, xr);
+  }
   float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < XL; ++k) {
@@ -458,6 +587,7 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
     }
     const int i = lane + 64 * k;
     *reinterpret_cast<float4*>(&xs[i >> 4][4 * (i & 15)]) = v;
+    if constexpr (ATTN) *reinterpret_cast<float4*>(&xc[4 * i]) = v;
   }
   __syncthreads();  // one wave: orders its LDS writes before its reads
   float x[64];
@@ -506,7 +636,8 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p) {
 #pragma unroll
     for (int hv = 0; hv < NH; ++hv) {
       if (!is_finite(v[hv]))
-        v[hv] = row_dot(W + (n + (hv ? p.swiglu_f : 0u)) * row_bytes, X, p.norm_alpha, p.K);
+        v[hv] = row_dot(W + (n + (hv ? p.swiglu_f : 0u)) * row_bytes, ATTN ? xc : X,
+                        p.norm_alpha, p.K);
       v[hv] *= inv;
     }
     float o = v[0];
@@ -908,7 +1039,7 @@ int launch_vec(const Q4kGemmParams& p, uint32_t nout, hipStream_t stream) {
                                            : q4k_vec_kernel<XL, R, false, true>)
                            : (p.norm_alpha ? q4k_vec_kernel<XL, R, true, false>
                                            : q4k_vec_kernel<XL, R, false, false>);
-  hipLaunchKernelGGL(kernel, grid, block, 0, stream, p);
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, p, NoAttention{});
   STS_HIP(hipGetLastError());
   return STS_OK;
 }
@@ -977,6 +1108,20 @@ int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
 }
 
 }  // namespace
+
+int launch_q4k_attention(const Q4kGemmParams& p, const DepthAttention& a, hipStream_t stream) {
+  if (p.M == 0 || p.M > 2 || p.N == 0 || p.Z != 1 || p.K == 0 || p.K % kQ4kBlockWeights != 0 ||
+      p.K > 1024 || p.swiglu_f || p.norm_alpha || a.len == 0 || a.len > a.max_len)
+    return fail(STS_ERR_INVALID, "attention and projection M=%u N=%u K=%u len=%u of %u", p.M, p.N,
+                p.K, a.len, a.max_len);
+  if ((uint64_t)a.max_len * p.K * sizeof(float) > 0x7FFFFFF0ull)
+    return fail(STS_ERR_INVALID, "cache of %u slots too large", a.max_len);
+  const dim3 grid((p.N + 3) / 4, p.M), block(64);
+  hipLaunchKernelGGL((q4k_vec_kernel<4, 1, false, false, DepthAttention>), grid, block, 0, stream,
+                     p, a);
+  STS_HIP(hipGetLastError());
+  return STS_OK;
+}
 
 int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   // Every check runs before anything is launched.

@@ -408,6 +408,39 @@ def test_depformer_chain_edge_cases(gpu, top_k):
     eng.close()
 
 
+@pytest.mark.parametrize("dim,heads,steps,slots", [
+    (256, 4, 5, 5), (512, 4, 4, 6), (768, 12, 9, 11), (1024, 16, 16, 16), (1280, 20, 4, 4)])
+def test_depformer_few_streams_as_many(gpu, dim, heads, steps, slots):
+    """One and two streams (attention inside the output projection for heads of
+    64 and dims up to 1024) against the same streams in a batch of three (a
+    launch each): the f32 sums differ in order only, 1e-5 of the logits' scale
+    over the two layers; a stream with an infinite input gives NaN in both."""
+    cfg = dict(CFG, dim=dim, num_heads=heads, num_steps=steps, kv_max_len=slots, num_layers=2,
+               num_audio_emb=steps - 1)
+    w = oracle.DepformerWeights.synthetic(cfg, seed=dim)
+    th, text, rand, pt, npn = _inputs(cfg, 3, 11)
+    th[2, 5] = np.inf
+    npn[:] = 0
+    eng = sts_attn.DepthEngine(_config(cfg), _device_weights(w), max_batch=3)
+
+    def run(rows):
+        lg = torch.empty((steps, len(rows), cfg["out_vocab"]), device="cuda")
+        tok = eng.generate(dev(th[rows]), dev(text[rows].view(np.int32)), 1.0, 1, 1.0,
+                           dev(rand[rows]), dev(pt[rows].view(np.int32)),
+                           dev(npn[rows].view(np.int32)), logits=lg)
+        return host(tok).view(np.uint32), host(lg)
+
+    tok3, lg3 = run([0, 1, 2])
+    assert np.isnan(lg3[0, 2]).all()
+    scale = np.abs(lg3[:, :2]).max()
+    for rows in ([0], [0, 1], [1], [2], [2, 1]):
+        tok, lg = run(rows)
+        np.testing.assert_array_equal(tok, tok3[rows])
+        np.testing.assert_array_equal(np.isnan(lg), np.isnan(lg3[:, rows]))
+        assert np.nanmax(np.abs(lg - lg3[:, rows]), initial=0) <= 1e-5 * scale
+    eng.close()
+
+
 @pytest.fixture(scope="module")
 def full_model():
     cfg = {f: getattr(sts_attn.DepformerConfig.personaplex(), f)
