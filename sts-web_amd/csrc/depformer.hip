@@ -168,10 +168,16 @@ __device__ __forceinline__ uint32_t count_above(const uint64_t* L, uint64_t x) {
 // NJ * 256 >= V.
 
 // Bound on how far the sampler's wave-scan running total can be from the
-// shader's single-lane one: each is within about 2K ulps of 1 of the exact
-// total (positive terms, K <= 256: 2 * 256 * 2^-24 = 3.1e-5), so they differ
-// by less than 6.2e-5 < 2^-13.
-constexpr float kDrawSlack = 1.0f / 8192.0f;
+// shader's single-lane one, both of positive terms that add up to 1, with
+// u = 2^-24: the shader's sum is within (K - 1) u of the exact one, its
+// quotients within u and its running total within another (K - 1) u; the
+// scan's sum (a tree) is within 8 u, its quotients u, its running total 12 u.
+// Together (2 K + 20) u.  A draw nearer to a boundary goes the slow way: of 64
+// streams drawing from 250 about every second launch has one, where a slack of
+// 2^-13 sent some stream of nearly every launch there.  With the slow way's two
+// chains freed of their LDS round trips and comparisons: 18.0 -> 13.8 us a
+// launch (10.9 with one stream).
+__device__ __forceinline__ float draw_slack(uint32_t K) { return (float)(2 * K + 64) * 0x1p-24f; }
 
 template <int NJ>
 __global__ __launch_bounds__(256) void sample_topk_kernel(const SampleParams p) {
@@ -187,7 +193,7 @@ __global__ __launch_bounds__(256) void sample_topk_kernel(const SampleParams p) 
   __shared__ uint64_t sbuf[2 * kMaxTopK];
   __shared__ uint32_t slot_idx[kMaxTopK];  // replayed selection: slot -> logit index
   __shared__ uint32_t s_tie[2];            // keys >= the K-th, any equal neighbours
-  __shared__ __align__(16) float cumv[kMaxTopK];  // the scan's running totals, then the weights
+  __shared__ __align__(16) float cumv[kMaxTopK];  // the scan's running totals, then the shader's
   static_assert(kMaxTopK == 256, "one key per thread in the ranking sort");
   const uint32_t tid = threadIdx.x, b = blockIdx.x, V = p.V;
   const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -418,10 +424,10 @@ __global__ __launch_bounds__(256) void sample_topk_kernel(const SampleParams p) 
   if (tid < 64) {
     // The cumulative draw (:212-221).  Wave 0: lane l holds values 4l..4l+3;
     // the sum and the running total come from a wave scan, a different f32
-    // order from the shader's single-lane loop, less than kDrawSlack away
-    // from it.  The scan's pick is therefore the shader's whenever rand lies
-    // further than kDrawSlack from the boundaries around it; otherwise lane 0
-    // redoes the shader's loop.
+    // order from the shader's single-lane loop, less than the slack away from
+    // it.  The scan's pick is therefore the shader's whenever rand lies further
+    // than that from the boundaries around it; otherwise lane 0 redoes the
+    // shader's loop.
     float e[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) e[c] = 4 * tid + c < K ? ev[4 * tid + c] : 0.f;
@@ -460,57 +466,81 @@ __global__ __launch_bounds__(256) void sample_topk_kernel(const SampleParams p) 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     // Certain when rand sits clear of the pick's upper boundary (or, with no
     // hit, of the last total) and of its lower one.
-    const bool sure = hits ? (rnd < cumv[pick] - kDrawSlack &&
-                              (pick == 0 || rnd >= cumv[pick - 1] + kDrawSlack))
-                           : rnd >= cumv[K - 1] + kDrawSlack;
+    const float slack = draw_slack(K);
+    const bool sure = hits ? (rnd < cumv[pick] - slack &&
+                              (pick == 0 || rnd >= cumv[pick - 1] + slack))
+                           : rnd >= cumv[K - 1] + slack;
     if (!sure) {
       // The shader's order: the sum in slot order, each weight divided by
-      // it, the running total in slot order.  Both chains run on lane 0 over
-      // 16 values at a time from LDS (the loads ahead of the additions; the
-      // slots past K hold +0, which leaves a sum unchanged), the divisions on
-      // every lane in between.
+      // it, the running total in slot order.  Both chains of additions run on
+      // lane 0, 16 values at a time from LDS with the next 16 on their way (the
+      // slots past K hold +0, which leaves a sum unchanged); the divisions and
+      // the comparisons with rand take every lane.
+      auto ld = [&](const float* v, uint32_t j, float4 (&t)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t[i] = *reinterpret_cast<const float4*>(v + j + 4 * i);
+      };
+      auto wave_sync = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      };
       float sq = 0.f;
       if (tid == 0) {
+        float4 t[4], nx[4];
+        ld(ev, 0, t);
+#pragma unroll 2
         for (uint32_t j0 = 0; j0 < K; j0 += 16) {
-          float4 t[4];
+          ld(ev, min(j0 + 16, kMaxTopK - 16u), nx);
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) t[q4] = *reinterpret_cast<const float4*>(&ev[j0 + 4 * q4]);
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            sq = sq + t[q4].x;
-            sq = sq + t[q4].y;
-            sq = sq + t[q4].z;
-            sq = sq + t[q4].w;
+          for (int i = 0; i < 4; ++i) {
+            sq = sq + t[i].x;
+            sq = sq + t[i].y;
+            sq = sq + t[i].z;
+            sq = sq + t[i].w;
+            t[i] = nx[i];
           }
         }
       }
       sq = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sq)));
 #pragma unroll
       for (int c = 0; c < 4; ++c) cumv[4 * tid + c] = e[c] / sq;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      uint32_t pk = K - 1;
+      wave_sync();
+      uint32_t done = 0;  // running totals in cumv
       if (tid == 0) {
         float cum = 0.f;
-        bool found = false;
-        for (uint32_t j0 = 0; j0 < K && !found; j0 += 16) {
-          float4 t[4];
+        float4 t[4], nx[4];
+        ld(cumv, 0, t);
+#pragma unroll 2
+        for (; done < K; done += 16) {
+          if (done > 0 && rnd < cum) break;
+          ld(cumv, min(done + 16, kMaxTopK - 16u), nx);
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) t[q4] = *reinterpret_cast<const float4*>(&cumv[j0 + 4 * q4]);
-          const float w[16] = {t[0].x, t[0].y, t[0].z, t[0].w, t[1].x, t[1].y, t[1].z, t[1].w,
-                               t[2].x, t[2].y, t[2].z, t[2].w, t[3].x, t[3].y, t[3].z, t[3].w};
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            cum = cum + w[i];
-            if (!found && j0 + i < K && rnd < cum) {
-              pk = j0 + i;
-              found = true;
-            }
+          for (int i = 0; i < 4; ++i) {
+            float4 o;
+            cum = o.x = cum + t[i].x;
+            cum = o.y = cum + t[i].y;
+            cum = o.z = cum + t[i].z;
+            cum = o.w = cum + t[i].w;
+            *reinterpret_cast<float4*>(cumv + done + 4 * i) = o;
+            t[i] = nx[i];
           }
         }
       }
-      pick = __builtin_amdgcn_readfirstlane(pk);
+      wave_sync();
+      done = min((uint32_t)__builtin_amdgcn_readfirstlane(done), K);
+      const float4 cm = *reinterpret_cast<const float4*>(cumv + 4 * tid);
+      const float cs[4] = {cm.x, cm.y, cm.z, cm.w};
+      first = 4;
+#pragma unroll
+      for (int c = 3; c >= 0; --c)
+        if (4 * tid + c < done && rnd < cs[c]) first = c;
+      const uint64_t found = __ballot(first < 4);
+      pick = K - 1;
+      if (found) {
+        const int lane0 = __builtin_ctzll(found);
+        pick = 4 * lane0 + __shfl(first, lane0, 64);
+      }
     }
     if (tid == 0) {
       // The draw picked a rank (the values by rank, and so the draw, are the
