@@ -291,14 +291,19 @@ __global__ __launch_bounds__(256 * KSPLIT) void prefill_kernel(const PrefillPara
 #pragma unroll
       for (int a = 0; a < QN; ++a)
         kf[a] = *reinterpret_cast<const float4*>(&sm.ks[krow * KP + a * 16 + g * 4]);
-      s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      // Two sums of half the dimensions each: what a score is off by is most
+      // of what a result is off by (300 queries after 1100 cached, against 64
+      // bits: 4.9e-7 with one sum, 3.7e-7 with two; 103.6-104.5 and 103.9 us).
+      floatx4 half[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int a = 0; a < QN; ++a) {
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].x, qop[a].x, s[t], 0, 0, 0);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].y, qop[a].y, s[t], 0, 0, 0);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].z, qop[a].z, s[t], 0, 0, 0);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].w, qop[a].w, s[t], 0, 0, 0);
+        floatx4& sh = half[a < QN / 2];
+        sh = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].x, qop[a].x, sh, 0, 0, 0);
+        sh = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].y, qop[a].y, sh, 0, 0, 0);
+        sh = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].z, qop[a].z, sh, 0, 0, 0);
+        sh = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a].w, qop[a].w, sh, 0, 0, 0);
       }
+      s[t] = half[0] + half[1];
     }
   
 
