@@ -1348,7 +1348,8 @@ int launch_ws(const PrefillParams& p, hipStream_t stream) {
 // average tile, a block's worth of start and merge per workgroup and a little
 // for each record of the fold.  24 queries after 2500 cached: 8 splits 36.7 us
 // (4: 56.8); 300 after 1100: 3 splits 84 (4: 92); 130 after 2500: 5 splits 98
-// (4: 111); 512 after 256: 2 splits 55.9 (3: 60.9).
+// (4: 111); 512 after 256: 2 splits 55.9 (3: 60.9).  (Measured when one record
+// was folded after the other; each is 1 to 2.6 us less with four at once.)
 uint32_t f32_splits(uint32_t S, uint32_t H, uint32_t len) {
   const uint32_t tiles = H * ((S + kBQ - 1) / kBQ), cus = (uint32_t)device_cu_count();
   const uint32_t longest = (len + kBK - 1) / kBK;
