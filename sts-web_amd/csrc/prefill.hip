@@ -605,7 +605,8 @@ __device__ __forceinline__ void ws_signal(uint32_t* ctr, int lane) {
 // [H][M][D] bf16, rounded to nearest even as the f32 path rounds them in its
 // producers), so the producers move half the bytes and convert nothing; the
 // stages, and therefore the result, are those of the f32-input kernel.
-template <int D, bool SPLIT, bool KV16 = false>
+// SPLITS: the tile's key blocks are shared by several workgroups (ws_splits).
+template <int D, bool SPLIT, bool KV16, bool SPLITS>
 __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) {
   static_assert(!(SPLIT && KV16), "the split variant needs the f32 rows");
   using Stage = WsStage<D, SPLIT>;
@@ -640,23 +641,41 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
   const uint32_t q_last = min(p.S, (qt + 1) * QT) - 1;
   const uint32_t kend = min(p.len, base_w + q_last + 1);
   // This workgroup's share of the tile's key blocks: all of them, or with
-  // several splits (few tiles in the launch) blocks [blk0, blk0 + nblk).
+  // SPLITS blocks [blk0, blk0 + own).
   const uint32_t nb_tile = (kend + KB - 1) / KB;
-  const uint32_t ns = min(p.nsplit, nb_tile), split = blockIdx.z;
+  const uint32_t ns = SPLITS ? min(p.nsplit, nb_tile) : 1u, split = SPLITS ? blockIdx.z : 0u;
   if (split >= ns) return;  // the tile has fewer blocks than splits
   const uint32_t blk0 = split * nb_tile / ns;
-  const uint32_t nblk = (split + 1) * nb_tile / ns - blk0;
+  const uint32_t own = (split + 1) * nb_tile / ns - blk0;
   // Visit order of the key blocks: the tiles within two blocks of the
   // launch's longest take theirs last to first.  They then start on blocks
   // few other tiles read and end on the ones every tile of the head has
   // already brought into L2 (512 queries after 256 cached, f32 K/V: 20.0 ->
   // 19.0 us per layer; the same order on the mirror path keeps its result
   // bit-identical to this one's; the split kernel, 0.25 us slower with it,
-  // keeps the forward order).  Step i of producers and consumers handles
-  // block blk(i); steps past the last block stay past it (zero loads).
+  // keeps the forward order).
   const uint32_t maxblk = (p.len + KB - 1) / KB;
-  const bool reverse = !SPLIT && p.nsplit == 1 && nblk + 2 >= maxblk;
-  auto blk = [&](uint32_t i) { return reverse && i < nblk ? nblk - 1 - i : blk0 + i; };
+  const bool reverse = !SPLIT && nb_tile + 2 >= maxblk;
+  // The weights are rounded to bf16 relative to the softmax base, so a split
+  // with a base of its own would round them otherwise than one workgroup
+  // walking the whole tile (2.3e-3 apart, either 3.3e-3 from 64 bits).  Every
+  // split therefore first takes the base from the scores of the blocks that
+  // the whole walk visits first, as far as every query has a key in both
+  // slices: one block forward, up to three backward.  The split that owns
+  // those blocks has them first anyway.
+  uint32_t npre = 0;
+  if (SPLITS && split != (reverse ? ns - 1 : 0u)) {
+    const uint32_t low = base_w + qt * QT;  // last key of the tile's first query
+    npre = reverse ? nb_tile - (low >= 32 ? (low - 32) / KB : 0u) : 1u;
+  }
+  // Step i of producers and consumers handles block blk(i); steps past the
+  // last block stay past it (zero loads).
+  const uint32_t nblk = npre + own;
+  auto blk = [&](uint32_t i) {
+    if (SPLITS && i < npre) return reverse ? nb_tile - 1 - i : i;
+    const uint32_t j = i - npre;
+    return reverse && j < own ? blk0 + own - 1 - j : blk0 + j;
+  };
   if (tid < NS) {
     filled[tid] = 0;
     vfilled[tid] = 0;
@@ -669,10 +688,10 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
   // the longest tiles, which set the kernel's end, start under less HBM
   // traffic; the shorter ones still finish first (measured at 512 queries
   // after 256 cached: 17.6 -> 16.5 us per layer).
-  if (KV16 && p.start_stagger) {
+  if (KV16 && !SPLITS && p.start_stagger) {
     // At most 16 blocks' worth: a bounded head start for the long tiles,
     // however many blocks a launch has.
-    const uint32_t n = min(maxblk - nblk, 16u) * p.start_stagger;
+    const uint32_t n = min(maxblk - nb_tile, 16u) * p.start_stagger;
     for (uint32_t i = 0; i < n; ++i) __builtin_amdgcn_s_sleep(2);
   }
 
@@ -722,9 +741,11 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
       uint32_t slot0 = p.start + kb;
       slot0 = slot0 >= p.M ? slot0 - p.M : slot0;
       uint32_t vo[NL];
-      uint32_t so = 0;
-      if (kb + KB <= lim && slot0 + KB <= p.M) {
-        so = slot0 * ROWB;
+      // The steps that only give the base read no V.
+      const uint32_t vlim = SPLITS && b < npre ? 0u : lim;
+      const bool whole = kb + KB <= vlim && slot0 + KB <= p.M;
+      const uint32_t so = whole ? slot0 * ROWB : 0u;
+      if (whole) {
 #pragma unroll
         for (int i = 0; i < KP16; ++i) vo[i] = k_row(i) * ROWB + c8 * 16;
 #pragma unroll
@@ -732,18 +753,18 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
 #pragma unroll
           for (int r4 = 0; r4 < 4; ++r4) vo[KP16 + 4 * i + r4] = v_row(i, r4) * ROWB + c8 * 16;
       } else {
-        auto off = [&](uint32_t r) {
+        auto off = [&](uint32_t r, uint32_t end) {
           const uint32_t row = kb + r;
           uint32_t slot = slot0 + r;
           slot = min(slot, slot - p.M);  // wrap (slot < 2M)
-          return row < lim ? slot * ROWB + c8 * 16 : 0xFFFFFFF0u;
+          return row < end ? slot * ROWB + c8 * 16 : 0xFFFFFFF0u;
         };
 #pragma unroll
-        for (int i = 0; i < KP16; ++i) vo[i] = off(k_row(i));
+        for (int i = 0; i < KP16; ++i) vo[i] = off(k_row(i), lim);
 #pragma unroll
         for (int i = 0; i < VP16; ++i)
 #pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) vo[KP16 + 4 * i + r4] = off(v_row(i, r4));
+          for (int r4 = 0; r4 < 4; ++r4) vo[KP16 + 4 * i + r4] = off(v_row(i, r4), vlim);
       }
 #pragma unroll
       for (int i = 0; i < KP16; ++i)
@@ -867,9 +888,11 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
       uint32_t slot0 = p.start + kb;
       slot0 = slot0 >= p.M ? slot0 - p.M : slot0;
       uint32_t vo[NL];
-      uint32_t so = 0;
-      if (kb + KB <= lim && slot0 + KB <= p.M) {
-        so = slot0 * ROWB;
+      // The steps that only give the base read no V.
+      const uint32_t vlim = SPLITS && b < npre ? 0u : lim;
+      const bool whole = kb + KB <= vlim && slot0 + KB <= p.M;
+      const uint32_t so = whole ? slot0 * ROWB : 0u;
+      if (whole) {
 #pragma unroll
         for (int i = 0; i < KPER; ++i) vo[i] = k_row(i) * ROWB + d4 * 16;
 #pragma unroll
@@ -877,18 +900,18 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
 #pragma unroll
           for (int r4 = 0; r4 < 4; ++r4) vo[KPER + 4 * i + r4] = v_row(i, r4) * ROWB + d4 * 16;
       } else {
-        auto off = [&](uint32_t r) {
+        auto off = [&](uint32_t r, uint32_t end) {
           const uint32_t row = kb + r;
           uint32_t slot = slot0 + r;
           slot = min(slot, slot - p.M);  // wrap (slot < 2M)
-          return row < lim ? slot * ROWB + d4 * 16 : 0xFFFFFFF0u;
+          return row < end ? slot * ROWB + d4 * 16 : 0xFFFFFFF0u;
         };
 #pragma unroll
-        for (int i = 0; i < KPER; ++i) vo[i] = off(k_row(i));
+        for (int i = 0; i < KPER; ++i) vo[i] = off(k_row(i), lim);
 #pragma unroll
         for (int i = 0; i < VPER; ++i)
 #pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) vo[KPER + 4 * i + r4] = off(v_row(i, r4));
+          for (int r4 = 0; r4 < 4; ++r4) vo[KPER + 4 * i + r4] = off(v_row(i, r4), vlim);
       }
 #pragma unroll
       for (int i = 0; i < KPER; ++i)
@@ -1067,10 +1090,8 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
       }
       return sc;
     };
-    // Mask, online softmax and O^T += V^T P^T of block i; releases its stage.
-    auto finish_block = [&](uint32_t i, f32x16 sc, float mb) {
-      const uint32_t s = i % NS;
-      const Stage& sg = st[s];
+    // Masks block i's scores and moves the base if they need it.
+    auto take_base = [&](uint32_t i, f32x16& sc, float mb) {
       const uint32_t k0 = blk(i) * KB + ks * 32;
       const bool unmasked = k0 + 31 < kend && k0 + 31 <= w_first;
       if (!unmasked) {
@@ -1100,6 +1121,12 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
 #pragma unroll
         for (int v = 0; v < 16; ++v) nbase[v] = -mbase;
       }
+    };
+    // Mask, online softmax and O^T += V^T P^T of block i; releases its stage.
+    auto finish_block = [&](uint32_t i, f32x16 sc, float mb) {
+      const uint32_t s = i % NS;
+      const Stage& sg = st[s];
+      take_base(i, sc, mb);
       // The weights exp2(s - m): sc already less mb, so only a moved base
       // needs a subtraction.
       const float dm = m - mb;
@@ -1164,7 +1191,13 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
     // (Consumers one block ahead, the next block's score MFMAs issued before
     // this block's softmax, measured slower once the softmax lost the
     // subtraction and the row-sum additions: mirror 16.9 against 16.1 us.)
-    for (uint32_t i = 0; i < nblk; ++i) {
+    for (uint32_t i = 0; i < npre; ++i) {
+      const float mb = mbase;
+      f32x16 sc = s_block(i);
+      take_base(i, sc, mb);
+      ws_signal(&released[i % NS], lane);
+    }
+    for (uint32_t i = npre; i < nblk; ++i) {
       const float mb = mbase;
       finish_block(i, s_block(i), mb);
     }
@@ -1186,7 +1219,7 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
     dst[OT * 16 + 1] = lsum;
   }
   __syncthreads();
-  if (p.nsplit > 1) {
+  if constexpr (SPLITS) {
     // Publish the split's unnormalised rows: per query group OT * 4 float4 and
     // (max, sum) of every lane, whole kilobytes per store.
     constexpr int RV = OT * 4;                     // float4 of a lane
@@ -1296,20 +1329,27 @@ __global__ __launch_bounds__(512) void prefill_ws_kernel(const PrefillParams p) 
 // chunks) leaves most CUs idle while each tile walks a long window alone, so
 // its blocks are dealt to as many workgroups as there are CUs, at least two
 // blocks each.  The splits' rows meet in memory (about 4 us), so the window
-// must shorten by six blocks or more for it (0.9 us a block).
-uint32_t ws_splits(uint32_t S, uint32_t H, uint32_t len) {
+// must shorten by six blocks or more for it.  The bf16 kernel (0.75 us a block)
+// pays for the blocks that only give the base on top, two for up to 32 queries
+// and three for more, and a little for every further tile; the split kernel
+// (1.5 us) has one.  32 heads, bf16 rows, one split against several: 24 queries
+// at the end of 9 blocks 11.1 and 11.1 us, of 11 12.6 and 11.6, of 18 17.8 and
+// 13.9; 100 queries of 12 blocks 14.2 and 13.7, f32 rows 14.7 and 15.0; split
+// kernel, 24 queries of 8 blocks 17.7 and 13.6.
+uint32_t ws_splits(uint32_t S, uint32_t H, uint32_t len, bool split_planes) {
   const uint32_t tiles = H * ((S + 63) / 64), nb = (len + kWsKB - 1) / kWsKB;
   const uint32_t ns = std::min({(uint32_t)device_cu_count() / tiles, kMaxWsSplits, nb / 2});
-  return ns > 1 && nb - (nb + ns - 1) / ns >= 6 ? ns : 1u;
+  const uint32_t base = split_planes ? 0 : 2 + std::min((S - 1) / 32, 2u);
+  return ns > 1 && nb >= (nb + ns - 1) / ns + base + 6 ? ns : 1u;
 }
 
 // The workspace of those splits; *nsplit falls back to 1 where it is not to be
 // had (the stream is being captured and it would have to grow).
 template <int D>
-int ws_workspace(uint32_t S, uint32_t H, uint32_t len, hipStream_t stream, uint32_t* nsplit,
-                 Workspace** out) {
+int ws_workspace(uint32_t S, uint32_t H, uint32_t len, bool split_planes, hipStream_t stream,
+                 uint32_t* nsplit, Workspace** out) {
   *out = nullptr;
-  *nsplit = ws_splits(S, H, len);
+  *nsplit = ws_splits(S, H, len, split_planes);
   if (*nsplit <= 1) return STS_OK;
   const uint32_t tiles = H * ((S + 63) / 64);
   if (int rc = try_workspace(stream, (size_t)tiles * *nsplit * 2 * 64 * (D / 2 + 4), tiles, out))
@@ -1326,7 +1366,7 @@ int launch_ws(const PrefillParams& p, hipStream_t stream) {
     return fail(STS_ERR_INVALID, "max_len %u too large for one head's buffer resource", p.M);
   PrefillParams q = p;
   Workspace* ws = nullptr;
-  if (int rc = ws_workspace<D>(p.S, p.H, p.len, stream, &q.nsplit, &ws)) return rc;
+  if (int rc = ws_workspace<D>(p.S, p.H, p.len, SPLIT, stream, &q.nsplit, &ws)) return rc;
   if (ws) {
     q.part = ws->part;
     q.counters = ws->counters;
@@ -1336,8 +1376,12 @@ int launch_ws(const PrefillParams& p, hipStream_t stream) {
                             (uint64_t)p.H * nqt <= (uint64_t)device_cu_count()
                         ? 10u
                         : 0u;
-  hipLaunchKernelGGL((prefill_ws_kernel<D, SPLIT, KV16>), dim3(p.H, nqt, q.nsplit), dim3(512), 0,
-                     stream, q);
+  if (q.nsplit > 1)
+    hipLaunchKernelGGL((prefill_ws_kernel<D, SPLIT, KV16, true>), dim3(p.H, nqt, q.nsplit),
+                       dim3(512), 0, stream, q);
+  else
+    hipLaunchKernelGGL((prefill_ws_kernel<D, SPLIT, KV16, false>), dim3(p.H, nqt), dim3(512), 0,
+                       stream, q);
   STS_HIP(hipGetLastError());
   return STS_OK;
 }
@@ -1473,9 +1517,11 @@ int reserve_prefill(uint32_t S, uint32_t H, uint32_t len, uint32_t head_dim, int
     return reserve_decode(S, H, head_dim, len, stream);  // launch_prefill_by_decode's plan
   uint32_t nsplit = 1;
   Workspace* ws = nullptr;
-  if (bf16_rows || precision != STS_PREC_F32)
-    return head_dim == 128 ? ws_workspace<128>(S, H, len, stream, &nsplit, &ws)
-                           : ws_workspace<64>(S, H, len, stream, &nsplit, &ws);
+  if (bf16_rows || precision != STS_PREC_F32) {
+    const bool split = precision == STS_PREC_F32_SPLIT_BF16;
+    return head_dim == 128 ? ws_workspace<128>(S, H, len, split, stream, &nsplit, &ws)
+                           : ws_workspace<64>(S, H, len, split, stream, &nsplit, &ws);
+  }
   return head_dim == 128 ? f32_workspace<128>(S, H, len, stream, &nsplit, &ws)
                          : f32_workspace<64>(S, H, len, stream, &nsplit, &ws);
 }

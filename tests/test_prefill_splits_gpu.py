@@ -11,6 +11,7 @@ import oracle
 import sts_attn
 from cases import prefill_inputs, scale_for
 from test_prefill_gpu import TOL_F32, dev, host, run, tol
+from test_workspace_gpu import _stream_pool, fresh_stream  # noqa: F401 (fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +85,38 @@ def test_grouped_heads_split(gpu):
         c.update(rows(k), rows(v))
         outs.append(host(c.prefill(dev(q), new(k), new(v), scale_for(D), F32)))
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+# H, D, M, cached rows, chunk rows, first slot: short chunks whose last block
+# leaves a key slice empty, wrapped windows, and long chunks of few heads, where
+# a split's only block lies past the window of some of its tile's queries.
+@pytest.mark.parametrize("prec", [BF16, SPLIT])
+@pytest.mark.parametrize("H,D,M,cached,S,start", [
+    (32, 128, 3000, 2500, 24, 100), (4, 128, 1200, 1100, 1, 700), (8, 64, 900, 800, 65, 850),
+    (2, 128, 3000, 2930, 64, 2999), (1, 64, 800, 0, 800, 3), (2, 128, 1000, 30, 900, 970)])
+def test_splits_round_as_one(gpu, fresh_stream, H, D, M, cached, S, start, prec):
+    """The splits' weights are rounded relative to the base that one workgroup
+    walking the whole tile has, so a launch with splits differs from one without
+    (a captured one on a stream that has no workspace) by its f32 sums alone:
+    about 2^-22 of the result, and a weight next to a rounding boundary now and
+    then, where bases of each split's own are 2e-3 apart (bf16)."""
+    print(f"prefill H={H} D={D} cached={cached} S={S} start={start} prec={prec}", flush=True)
+    q, kc, vc = prefill_inputs(H + cached + S, H, D, M, cached, S, start)
+    scale = scale_for(D)
+    qd, kd, vd, out = dev(q), dev(kc), dev(vc), torch.empty((S, H, D), device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=fresh_stream):
+        sts_attn.prefill_attention(qd, kd, vd, start, cached + S, scale, prec, out=out,
+                                   stream=fresh_stream)
+    ref = oracle.prefill_f64(q, kc, vc, start, cached + S, scale)
+    split = host(sts_attn.prefill_attention(qd, kd, vd, start, cached + S, scale, prec))
+    assert np.abs(split - ref).max() < tol(prec)
+    for _ in range(2):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        one = host(out)
+        d = np.linalg.norm(split.astype(np.float64) - one) / np.linalg.norm(one)
+        print(f"  splits against one: {d:.2e}", flush=True)
+        assert d <= 5e-5
