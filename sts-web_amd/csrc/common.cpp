@@ -36,6 +36,45 @@ void clear_error() { g_last_error.clear(); }
 
 const char* last_error_cstr() { return g_last_error.c_str(); }
 
+namespace {
+
+// Makes ws hold at least the requested sizes; g_ws_mutex is held.  Growing
+// allocates new buffers (new counters zero-filled on the stream) and retires
+// the old ones without freeing them.
+int grow_workspace(Workspace& ws, hipStream_t stream, size_t part_floats, size_t n_counters) {
+  if (ws.part_floats >= part_floats && ws.n_counters >= n_counters) return STS_OK;
+  // Growth at least doubles, so the retired buffers never exceed the live ones.
+  auto grow = [](size_t want, size_t have, size_t round) {
+    const size_t n = std::max<size_t>(std::max(want, have < want ? 2 * have : have), 1);
+    return (n + round - 1) / round * round;
+  };
+  const size_t pf = grow(part_floats, ws.part_floats, 65536);
+  const size_t nc = grow(n_counters, ws.n_counters, 1024);
+  float* part = nullptr;
+  uint32_t* counters = nullptr;
+  if (hipMalloc(&part, pf * sizeof(float)) != hipSuccess)
+    return fail(STS_ERR_NOMEM, "workspace allocation of %zu bytes failed", pf * sizeof(float));
+  if (hipMalloc(&counters, nc * sizeof(uint32_t)) != hipSuccess) {
+    (void)hipFree(part);
+    return fail(STS_ERR_NOMEM, "workspace counter allocation failed");
+  }
+  // The counters start at zero; every launch leaves them at zero.
+  if (hipMemsetAsync(counters, 0, nc * sizeof(uint32_t), stream) != hipSuccess) {
+    (void)hipFree(part);
+    (void)hipFree(counters);
+    return fail(STS_ERR_HIP, "workspace counter initialisation failed");
+  }
+  if (ws.part) g_retired.push_back(ws.part);
+  if (ws.counters) g_retired.push_back(ws.counters);
+  ws.part = part;
+  ws.counters = counters;
+  ws.part_floats = pf;
+  ws.n_counters = nc;
+  return STS_OK;
+}
+
+}  // namespace
+
 int get_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Workspace** out) {
   int dev = 0;
   STS_HIP(hipGetDevice(&dev));
@@ -52,35 +91,9 @@ int get_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Wor
                   "split workspace of %zu floats / %zu counters needed while the stream is "
                   "being captured; run the call once on this stream before capturing it",
                   part_floats, n_counters);
-    // The old buffers are retired, not freed: kernels queued on the stream
-    // and graphs captured earlier keep using them.  Growth at least doubles,
-    // so the retired buffers never exceed the live ones.
-    auto grow = [](size_t want, size_t have, size_t round) {
-      const size_t n = std::max<size_t>(std::max(want, have < want ? 2 * have : have), 1);
-      return (n + round - 1) / round * round;
-    };
-    const size_t pf = grow(part_floats, ws.part_floats, 65536);
-    const size_t nc = grow(n_counters, ws.n_counters, 1024);
-    float* part = nullptr;
-    uint32_t* counters = nullptr;
-    if (hipMalloc(&part, pf * sizeof(float)) != hipSuccess)
-      return fail(STS_ERR_NOMEM, "workspace allocation of %zu bytes failed", pf * sizeof(float));
-    if (hipMalloc(&counters, nc * sizeof(uint32_t)) != hipSuccess) {
-      (void)hipFree(part);
-      return fail(STS_ERR_NOMEM, "workspace counter allocation failed");
-    }
-    // The counters start at zero; every launch leaves them at zero.
-    if (hipMemsetAsync(counters, 0, nc * sizeof(uint32_t), stream) != hipSuccess) {
-      (void)hipFree(part);
-      (void)hipFree(counters);
-      return fail(STS_ERR_HIP, "workspace counter initialisation failed");
-    }
-    if (ws.part) g_retired.push_back(ws.part);
-    if (ws.counters) g_retired.push_back(ws.counters);
-    ws.part = part;
-    ws.counters = counters;
-    ws.part_floats = pf;
-    ws.n_counters = nc;
+    // Retired, not freed: kernels queued on the stream and graphs captured
+    // earlier keep using the old buffers.
+    if (int rc = grow_workspace(ws, stream, part_floats, n_counters)) return rc;
   }
   *out = &ws;
   return STS_OK;
@@ -97,6 +110,48 @@ int try_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Wor
   (void)hipGetLastError();
   clear_error();
   return STS_OK;
+}
+
+namespace {
+// Map nodes stay where they are, so an entry's lock outlives g_ws_mutex.
+struct ScratchEntry {
+  std::mutex held;
+  Workspace ws;
+};
+std::map<std::pair<int, hipStream_t>, ScratchEntry> g_scratch;
+}  // namespace
+
+Scratch::Scratch(hipStream_t stream, size_t part_floats, size_t n_counters) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return;
+  ScratchEntry* e = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    e = &g_scratch[{dev, stream}];
+  }
+  std::unique_lock<std::mutex> held(e->held);
+  if (e->ws.part_floats < part_floats || e->ws.n_counters < n_counters) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    bool ok = hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (ok && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+      {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        ok = grow_workspace(e->ws, stream, part_floats, n_counters) == STS_OK;
+      }
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    } else {
+      ok = false;
+    }
+    if (!ok) {
+      (void)hipGetLastError();
+      clear_error();
+      return;
+    }
+  }
+  part = e->ws.part;
+  counters = e->ws.counters;
+  held_ = std::move(held);
 }
 
 namespace {

@@ -7,6 +7,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 
 #include "sts_attn.h"
@@ -52,6 +53,27 @@ int get_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Wor
 // captured, memory is short).  The allocation is made in relaxed capture mode,
 // so that it does not break a capture of another stream in progress.
 int try_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Workspace** out);
+
+// Memory through which the launches of one call hand data to one another, per
+// (device, stream) and apart from Workspace.  Its holder has it alone until it
+// goes out of scope, which it does once the call's last launch is enqueued:
+// calls of other host threads on the same stream wait for that, so that their
+// launches come after all of this call's and not between two of them.
+// part is null where the memory would have to grow and cannot (`stream` is
+// being captured, memory is short): the caller then takes its way without.
+// Growing happens in relaxed capture mode, so that it does not break a capture
+// of another stream in progress, and retires the old buffers as Workspace does.
+class Scratch {
+ public:
+  Scratch(hipStream_t stream, size_t part_floats, size_t n_counters);
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  float* part = nullptr;
+  uint32_t* counters = nullptr;  // zero between calls
+
+ private:
+  std::unique_lock<std::mutex> held_;
+};
 
 // Number of compute units of the current device (cached per device).
 int device_cu_count();

@@ -1044,10 +1044,9 @@ int launch_vec(const Q4kGemmParams& p, uint32_t nout, hipStream_t stream) {
   return STS_OK;
 }
 
-// Many rows: x split once into the workspace, then the 64 x 128 tiles, in
-// chunks of at most kTileRows rows so that the workspace stays bounded.
-// *done stays false where the workspace is not to be had (the stream is being
-// captured and it would have to grow, or memory is short).
+// Many rows: x split once into scratch memory, then the 64 x 128 tiles, in
+// chunks of at most kTileRows rows so that the scratch stays bounded.
+// *done stays false where the scratch is not to be had.
 constexpr uint32_t kTileRows = 1024;
 int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
   const uint32_t KB = p.K / 32, SB = p.K / kQ4kBlockWeights;
@@ -1060,12 +1059,10 @@ int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
   const uint32_t ksplit = std::max(1u, std::min(2 * cus / tiles, SB / 4));
   const size_t plane_floats = TilePlanes::floats(rows, KB);
   const size_t y_floats = ksplit > 1 ? (size_t)rows * p.N : 0;
-  Workspace* ws = nullptr;
-  if (int rc = try_workspace(stream, plane_floats + ksplit * y_floats, 0, &ws))
-    return rc;
-  if (!ws) return STS_OK;
-  const TilePlanes planes(ws->part, rows, KB);
-  float* part = ws->part + plane_floats;
+  const Scratch scratch(stream, plane_floats + ksplit * y_floats, 0);  // held to the last launch
+  if (!scratch.part) return STS_OK;
+  const TilePlanes planes(scratch.part, rows, KB);
+  float* part = scratch.part + plane_floats;
   for (uint32_t m0 = 0; m0 < p.M; m0 += kTileRows) {
     Q4kTileParams t;
     t.w = p.w[0];

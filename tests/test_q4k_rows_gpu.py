@@ -201,3 +201,41 @@ def test_rows_not_finite(gpu, M, N, K):
     if M > 3:
         d = got[3:] - x[3:].astype(np.float64) @ wt.T
         assert (np.abs(d) <= 1e-5 * q4k_bound(blocks, x[3:], N)).all()
+
+
+def test_threads_on_one_stream(gpu):
+    """Two host threads with products of many rows and one with prefills whose
+    key ranges are split, all on the one stream that torch gives every thread:
+    each result is that of the call alone, bit for bit."""
+    import threading
+
+    M, N, K, H, D, cached, S = 128, 4096, 4096, 8, 128, 1500, 24
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = sts_attn.Q4KTensor.from_q4k_bytes(oracle._random_q4k_scaled(11, N, K), (N, K))
+    xs = [torch.randn((M, K), generator=g, device="cuda") for _ in range(2)]
+    q = torch.randn((S, H, D), generator=g, device="cuda")
+    kc, vc = (torch.randn((H, cached + S, D), generator=g, device="cuda") for _ in range(2))
+    calls = [lambda: sts_attn.q4k_gemm(xs[0], w), lambda: sts_attn.q4k_gemm(xs[1], w),
+             lambda: sts_attn.prefill_attention(q, kc, vc, 0, cached + S, 0.09,
+                                                sts_attn.PREC_BF16_MFMA)]
+    alone = [c() for c in calls]
+    torch.cuda.synchronize()
+    start, got, errors = threading.Barrier(3), [[] for _ in calls], []
+
+    def work(i):
+        try:
+            start.wait()
+            for _ in range(40):
+                got[i].append(calls[i]())
+        except Exception as e:  # reported below, in the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(3):
+        assert all(torch.equal(y, alone[i]) for y in got[i]), i
