@@ -32,14 +32,24 @@
  *     only).  The reference shader takes any head_dim up to 128 and silently
  *     overflows beyond (shader_attention.wgsl:36, :66); here that is an
  *     error, and so is a head_dim that is not a multiple of 4.
- *   - Attention entry points use a per-(device, stream) workspace owned by the
+ *   - Decodes and f32 prefills use a per-(device, stream) workspace owned by the
  *     library for split-KV partial results.  It is allocated (hipMalloc) on the
  *     first call on a stream that needs it and grown when a larger launch needs
  *     more; replaced buffers are retired, not freed, so graphs captured earlier
  *     stay valid.  A call that would allocate or grow it while its stream is
- *     being captured into a HIP graph fails with STS_ERR_STATE: run the largest
- *     call once on the stream before capturing it.  Calls issued on the same
- *     stream are ordered; calls on different streams use different workspaces.
+ *     being captured into a HIP graph fails with STS_ERR_STATE (an f32 prefill
+ *     that finds room for fewer splits than it would take runs with those): run
+ *     the largest call once on the stream before capturing it.  A graph keeps
+ *     using the workspace of the stream it was captured on: its replays must not
+ *     overlap in time with replays of other graphs captured on that stream or
+ *     with calls on it.  Calls issued on the same stream, also from several host
+ *     threads, are ordered; calls on different streams use different workspaces.
+ *   - Q4_K products of many rows (sts_q4k_gemm, sts_q4k_matvec) and bf16 and
+ *     split-bf16 prefills of short chunks after long windows use other memory of
+ *     the library, per (device, stream) and allocated the same way, which a call
+ *     has to itself until its last launch is enqueued.  They do without it, more
+ *     slowly and with f32 sums in another order, where memory is short and
+ *     always while the stream is being captured: graphs share none of it.
  *   - Handles are not internally locked: use one handle from one host thread at
  *     a time (the reference's caches are !Sync, model.rs:483).
  */

@@ -123,7 +123,12 @@ std::map<std::pair<int, hipStream_t>, ScratchEntry> g_scratch;
 
 Scratch::Scratch(hipStream_t stream, size_t part_floats, size_t n_counters) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamIsCapturing(stream, &cap) != hipSuccess ||
+      cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return;
+  }
   ScratchEntry* e = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
@@ -131,17 +136,14 @@ Scratch::Scratch(hipStream_t stream, size_t part_floats, size_t n_counters) {
   }
   std::unique_lock<std::mutex> held(e->held);
   if (e->ws.part_floats < part_floats || e->ws.n_counters < n_counters) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    bool ok = hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    if (ok && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+    bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (ok) {
       {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
         ok = grow_workspace(e->ws, stream, part_floats, n_counters) == STS_OK;
       }
       (void)hipThreadExchangeStreamCaptureMode(&mode);
-    } else {
-      ok = false;
     }
     if (!ok) {
       (void)hipGetLastError();

@@ -59,10 +59,12 @@ int try_workspace(hipStream_t stream, size_t part_floats, size_t n_counters, Wor
 // goes out of scope, which it does once the call's last launch is enqueued:
 // calls of other host threads on the same stream wait for that, so that their
 // launches come after all of this call's and not between two of them.
-// part is null where the memory would have to grow and cannot (`stream` is
-// being captured, memory is short): the caller then takes its way without.
-// Growing happens in relaxed capture mode, so that it does not break a capture
-// of another stream in progress, and retires the old buffers as Workspace does.
+// part is null where the caller has to take its way without: while `stream` is
+// being captured, so that a graph shares no memory with another one or with
+// eager calls beside its replays and its result does not depend on what ran
+// before the capture, and where memory is short.  Growing happens in relaxed
+// capture mode, so that it does not break a capture of another stream in
+// progress, and retires the old buffers as Workspace does.
 class Scratch {
  public:
   Scratch(hipStream_t stream, size_t part_floats, size_t n_counters);

@@ -34,6 +34,7 @@
 // finished tiles' output from pushing those shared blocks out of L2.
 #include <algorithm>
 #include <cfloat>
+#include <optional>
 
 #include "coherent.hpp"
 #include "common.hpp"
@@ -1343,21 +1344,6 @@ uint32_t ws_splits(uint32_t S, uint32_t H, uint32_t len, bool split_planes) {
   return ns > 1 && nb >= (nb + ns - 1) / ns + base + 6 ? ns : 1u;
 }
 
-// The workspace of those splits; *nsplit falls back to 1 where it is not to be
-// had (the stream is being captured and it would have to grow).
-template <int D>
-int ws_workspace(uint32_t S, uint32_t H, uint32_t len, bool split_planes, hipStream_t stream,
-                 uint32_t* nsplit, Workspace** out) {
-  *out = nullptr;
-  *nsplit = ws_splits(S, H, len, split_planes);
-  if (*nsplit <= 1) return STS_OK;
-  const uint32_t tiles = H * ((S + 63) / 64);
-  if (int rc = try_workspace(stream, (size_t)tiles * *nsplit * 2 * 64 * (D / 2 + 4), tiles, out))
-    return rc;
-  if (!*out) *nsplit = 1;
-  return STS_OK;
-}
-
 template <int D, bool SPLIT, bool KV16 = false>
 int launch_ws(const PrefillParams& p, hipStream_t stream) {
   const uint32_t nqt = (p.S + 63) / 64;
@@ -1365,11 +1351,15 @@ int launch_ws(const PrefillParams& p, hipStream_t stream) {
   if ((uint64_t)p.M * D * sizeof(float) > 0x7FFFFFF0ull)
     return fail(STS_ERR_INVALID, "max_len %u too large for one head's buffer resource", p.M);
   PrefillParams q = p;
-  Workspace* ws = nullptr;
-  if (int rc = ws_workspace<D>(p.S, p.H, p.len, SPLIT, stream, &q.nsplit, &ws)) return rc;
-  if (ws) {
-    q.part = ws->part;
-    q.counters = ws->counters;
+  // The splits' records; one split where they are not to be had.
+  const uint32_t tiles = p.H * nqt;
+  std::optional<Scratch> scratch;  // held until the launch is enqueued
+  q.nsplit = ws_splits(p.S, p.H, p.len, SPLIT);
+  if (q.nsplit > 1) {
+    scratch.emplace(stream, (size_t)tiles * q.nsplit * 2 * 64 * (D / 2 + 4), tiles);
+    q.part = scratch->part;
+    q.counters = scratch->counters;
+    if (!q.part) q.nsplit = 1;
   }
   // A sleeping workgroup costs nothing only while no other waits for its CU.
   q.start_stagger = KV16 && !SPLIT && q.nsplit == 1 &&
@@ -1515,13 +1505,9 @@ int reserve_prefill(uint32_t S, uint32_t H, uint32_t len, uint32_t head_dim, int
   if (int rc = device_error_word(&err)) return rc;
   if (head_dim != 64 && head_dim != 128)
     return reserve_decode(S, H, head_dim, len, stream);  // launch_prefill_by_decode's plan
+  if (bf16_rows || precision != STS_PREC_F32) return STS_OK;  // has a way without its scratch
   uint32_t nsplit = 1;
   Workspace* ws = nullptr;
-  if (bf16_rows || precision != STS_PREC_F32) {
-    const bool split = precision == STS_PREC_F32_SPLIT_BF16;
-    return head_dim == 128 ? ws_workspace<128>(S, H, len, split, stream, &nsplit, &ws)
-                           : ws_workspace<64>(S, H, len, split, stream, &nsplit, &ws);
-  }
   return head_dim == 128 ? f32_workspace<128>(S, H, len, stream, &nsplit, &ws)
                          : f32_workspace<64>(S, H, len, stream, &nsplit, &ws);
 }

@@ -254,3 +254,57 @@ def test_current_stream_handle(gpu, where):
         g.replay()
         torch.cuda.synchronize()
     assert sts_attn._stream(a) == a.cuda_stream and sts_attn._stream(7) == 7
+
+
+@pytest.mark.parametrize("call", ["gemm", "prefill"])
+def test_graphs_share_no_scratch(gpu, fresh_stream, call):
+    """A product of many rows and a bf16 prefill of a short chunk, which run
+    without scratch memory inside a capture: captured on a stream that has run
+    them before they give the bits of a capture on one that has not, and their
+    replays on another stream are not disturbed by eager calls on the first."""
+    g = torch.Generator(device="cuda").manual_seed(17)
+    if call == "gemm":
+        M, N, K = 128, 4096, 4096
+        w = sts_attn.Q4KTensor.from_q4k_bytes(oracle._random_q4k_scaled(19, N, K), (N, K))
+        x, other = (torch.randn((M, K), generator=g, device="cuda") for _ in range(2))
+        out, out2 = (torch.empty((M, N), device="cuda") for _ in range(2))
+
+        def run(inp, out, s):
+            sts_attn.q4k_gemm(inp, w, out=out, stream=s)
+    else:
+        H, D, cached, S = 8, 128, 1500, 24
+        x, other = (torch.randn((S, H, D), generator=g, device="cuda") for _ in range(2))
+        kc, vc = (torch.randn((H, cached + S, D), generator=g, device="cuda") for _ in range(2))
+        out, out2 = (torch.empty((S, H, D), device="cuda") for _ in range(2))
+
+        def run(inp, out, s):
+            sts_attn.prefill_attention(inp, kc, vc, 0, cached + S, scale_for(D),
+                                       sts_attn.PREC_BF16_MFMA, out=out, stream=s)
+
+    def captured(s):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            run(x, out, s)
+        return graph
+
+    def replay(graph):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        return host(out).copy()
+
+    torch.cuda.synchronize()
+    want = replay(captured(fresh_stream))
+    run(other, out2, fresh_stream)
+    fresh_stream.synchronize()
+    graph = captured(fresh_stream)
+    np.testing.assert_array_equal(replay(graph), want)
+    for _ in range(5):
+        out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(4):
+            run(other, out2, fresh_stream)
+            graph.replay()  # on torch's current stream, beside the eager calls
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host(out), want)
