@@ -361,33 +361,35 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
 
 // One weight of a slot after the other is what a single row of x is worth: no
 // 16-row tile to fill.  The 64 weights of slot s of a row (iteration s % 4 of
-// super-block s / 4) against the lane's x values: the nibble in a byte's upper
-// half with its top bit flipped is 16 (q - 8) as a signed byte, so no offset has
-// to cancel (the min takes 8 d sc off again).
-__device__ __forceinline__ float slot_dot8(u32x4 hd, u32x4 qa, u32x4 qb, uint32_t j,
-                                           const float (&x)[64], float sl, float sh) {
+// super-block s / 4) against the lane's x values.  d*sc, dmin*mn and q*(d*sc)
+// are exact in f32, so one fma rounds the weight as the shader does, and a small
+// weight stays small under a large x: the quants' and the mins' shares summed
+// apart are two large terms there, whose roundings the difference keeps.
+__device__ __forceinline__ float slot_dot(u32x4 hd, u32x4 qa, u32x4 qb, uint32_t j,
+                                          const float (&x)[64]) {
   const float d = half_bits_to_float(hd.x), dmin = half_bits_to_float(hd.x >> 16);
   uint32_t scl, mnl, sch, mnh;
   scale_min(hd.y, hd.z, hd.w, j, scl, mnl);
   scale_min(hd.y, hd.z, hd.w, j + 1, sch, mnh);
+  const float d1 = d * (float)scl, m1 = dmin * (float)mnl;
+  const float d2 = d * (float)sch, m2 = dmin * (float)mnh;
   const uint32_t words[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-  float ql[4] = {0.f, 0.f, 0.f, 0.f}, qh[4] = {0.f, 0.f, 0.f, 0.f};
+  float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < 8; ++w) {
-    const uint32_t lo = ((words[w] << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
-    const uint32_t hi = (words[w] & 0xF0F0F0F0u) ^ 0x80808080u;
+    uint32_t lo = words[w] & 0x0F0F0F0Fu;
+    uint32_t hi = (words[w] >> 4) & 0x0F0F0F0Fu;
+    // Opaque to the optimiser, so each byte below is one v_cvt_f32_ubyte.
+    asm("" : "+v"(lo), "+v"(hi));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      ql[i] = __builtin_fmaf((float)(int8_t)(lo >> (8 * i)), x[4 * w + i], ql[i]);
-      qh[i] = __builtin_fmaf((float)(int8_t)(hi >> (8 * i)), x[32 + 4 * w + i], qh[i]);
+      const float wl = __builtin_fmaf((float)((lo >> (8 * i)) & 0xFFu), d1, -m1);
+      const float wh = __builtin_fmaf((float)((hi >> (8 * i)) & 0xFFu), d2, -m2);
+      a[i] = __builtin_fmaf(wl, x[4 * w + i], a[i]);
+      b[i] = __builtin_fmaf(wh, x[32 + 4 * w + i], b[i]);
     }
   }
-  const float d1 = d * (float)scl * 0.0625f, d2 = d * (float)sch * 0.0625f;  // exact
-  const float m1 = __builtin_fmaf(128.f, d1, -(dmin * (float)mnl));
-  const float m2 = __builtin_fmaf(128.f, d2, -(dmin * (float)mnh));
-  const float a = __builtin_fmaf(d1, (ql[0] + ql[1]) + (ql[2] + ql[3]), m1 * sl);
-  const float b = __builtin_fmaf(d2, (qh[0] + qh[1]) + (qh[2] + qh[3]), m2 * sh);
-  return a + b;
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3]));
 }
 
 // Decode attention of all heads (dim 64) of one stream over the slots 0..len-1
@@ -599,13 +601,6 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p, cons
     x[4 * j + 2] = t.z;
     x[4 * j + 3] = t.w;
   }
-  float sl[4] = {0.f, 0.f, 0.f, 0.f}, sh[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    sl[j & 3] += x[j];
-    sh[j & 3] += x[32 + j];
-  }
-  const float sxl = (sl[0] + sl[1]) + (sl[2] + sl[3]), sxh = (sh[0] + sh[1]) + (sh[2] + sh[3]);
   auto lanes_sum = [&](float v) {
     v += xchg<0>(v);
     v += xchg<1>(v);
@@ -631,7 +626,7 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p, cons
     float v[NH];
 #pragma unroll
     for (int hv = 0; hv < NH; ++hv)
-      v[hv] = lanes_sum(slot_dot8(hd[j][hv], qa[j][hv], qb[j][hv], 2 * (slot & 3u), x, sxl, sxh));
+      v[hv] = lanes_sum(slot_dot(hd[j][hv], qa[j][hv], qb[j][hv], 2 * (slot & 3u), x));
     if (s != 0 || n >= nout) continue;
 #pragma unroll
     for (int hv = 0; hv < NH; ++hv) {

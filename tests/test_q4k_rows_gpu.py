@@ -239,3 +239,58 @@ def test_threads_on_one_stream(gpu):
     assert not errors, errors
     for i in range(3):
         assert all(torch.equal(y, alone[i]) for y in got[i]), i
+
+
+def near_zero_blocks(seed, N, K, cols):
+    """Random Q4_K matrix whose even rows have dmin = 8 d and every min equal to
+    its scale, and whose weights in the given columns (one or more of each
+    super-block) are the ones nearest to zero: exactly zero in the even rows, less
+    than half a quant step in the others (where the min is within the quants'
+    range)."""
+    blk = oracle._random_q4k_scaled(seed, N, K).reshape(N, K // 256, 144).copy()
+    s = blk[..., 4:16]
+    even = slice(0, None, 2)
+    dm = np.float16(8 * float(blk[0, 0, :2].view(np.float16)[0]))
+    blk[even, :, 2:4] = np.array([dm]).view(np.uint8)
+    s[even, :, 4:8] = s[even, :, 0:4]
+    s[even, :, 8:12] = (s[even, :, 8:12] & 15) * 17
+    d = blk[..., 0:2].copy().view(np.float16)[..., 0].astype(np.float64)
+    dmin = blk[..., 2:4].copy().view(np.float16)[..., 0].astype(np.float64)
+    for c in cols:
+        b, j, i = c // 256, c // 32 % 8, c % 32
+        if j < 4:
+            sc, mn = s[:, b, j] & 63, s[:, b, 4 + j] & 63
+        else:
+            sc = (s[:, b, 4 + j] & 15) | (s[:, b, j - 4] >> 6 << 4)
+            mn = (s[:, b, 4 + j] >> 4) | (s[:, b, j] >> 6 << 4)
+        with np.errstate(divide="ignore", invalid="ignore"):
+            q = np.nan_to_num(np.rint(dmin[:, b] * mn / (d[:, b] * sc)), posinf=15)
+        q = q.clip(0, 15).astype(np.uint8)
+        byte = 16 + 32 * (j // 2) + i
+        old = blk[:, b, byte]
+        blk[:, b, byte] = (old & 0xF0) | q if j % 2 == 0 else (old & 0x0F) | (q << 4)
+    return blk.reshape(-1)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 515, 1024), (2, 301, 2304), (1, 130, 4096)])
+def test_small_weights_under_large_x(gpu, M, N, K):
+    """Channels of x up to 1e12 times the others at weights that are zero or
+    nearly: each output is within 2e-6 of sum |w x|, 33 roundings of f32 at that
+    size (a sum of thousands of terms of random sign stays below), with no
+    allowance for the mins.  Sums over quants and mins apart, or x held to fewer
+    bits of the largest value of its block, are off by far more."""
+    print(f"q4k large channels M={M} N={N} K={K}", flush=True)
+    cols = [256 * b + (37 * b + 11) % 256 for b in range(K // 256)]
+    blocks = near_zero_blocks(M + N + K, N, K, cols)
+    x = oracle.normal(N + 3 * M, (M, K))
+    for m in range(M):
+        x[m, cols] *= np.float32(10.0 ** (12 - m % 13))
+    wt = torch.from_numpy(oracle.q4k_dequant(blocks, N, K)).cuda().double()
+    assert (wt[::2, cols] == 0).all()
+    got = host(sts_attn.q4k_gemm(dev(x), sts_attn.Q4KTensor.from_q4k_bytes(blocks, (N, K))))
+    xd = dev(x).double()
+    ref = (xd @ wt.T.contiguous()).cpu().numpy()
+    size = (xd.abs() @ wt.abs().T.contiguous()).cpu().numpy()
+    worst = (np.abs(got - ref) / size).max()
+    print(f"  worst error over sum |w x|: {worst:.2e}", flush=True)
+    assert worst <= 2e-6
