@@ -1,22 +1,24 @@
-// q4k_gemm.hip -- Q4_K products for more than one row on the bf16 matrix cores (gfx950).
+// q4k_gemm.hip -- Q4_K products for more than one row on the f16 matrix cores (gfx950).
 //
 // Y[m][n] = sum_k W[n][k] X[m][k] with W in Q4_K (q4k_matmul with M > 1,
 // crates/sts-wasm/src/gguf.rs:810-897, and the depformer's projections,
 // depth_engine.rs:953-1360).  f32 results without f32 matrix instructions:
 //
-//   W = d*sc_j * q - dmin*mn_j per sub-block j of 32 weights, q in 0..15.  A
-//   bf16 holds q exactly, and every f32 x is exactly the sum of three bf16
-//   values: hi = x truncated to its top 16 bits, mid = (x - hi) truncated
-//   likewise, lo = x - hi - mid (24 = 8 + 8 + 8 significand bits, each
-//   difference exact).  So three v_mfma_f32_16x16x32_bf16 per sub-block give
-//   sum q*x with exact products and f32 accumulation; d*sc_j scales that sum
-//   in f32, and dmin*mn_j times the sub-block's sum of x is subtracted by one
-//   v_mfma_f32_16x16x4f32 per four sub-blocks.  The weights are never rounded
-//   (the f32 weight d*sc*q - dmin*mn of the shader rounds once).
+//   W = d*sc_j * (q - z_j) + rest_j per sub-block j of 32 weights, z_j the whole
+//   number of quant steps nearest to its min (zero_point).  sc_j * (q - z_j) is a
+//   whole number up to 945, exact in f16, and x, scaled by a power of two per row
+//   and block, is a sum of f16 values: three of them hold all its 24 bits.  So
+//   v_mfma_f32_16x16x32_f16 on x's parts, each with an accumulator of its own,
+//   give sum sc*(q - z)*x with exact products and f32 accumulation; d scales that
+//   sum in f32, and rest_j times the sub-block's sum of x is added by one
+//   v_mfma_f32_16x16x4f32 per four sub-blocks.  (Products of many rows still take
+//   z = 8 throughout, see there.)
 //   Against v_mfma_f32_16x16x4f32 on dequantised weights (one per 4 weights,
-//   32 clocks) this takes 48 + 8 matrix clocks instead of 256 per 16x16
-//   outputs and 32 weights, and the nibbles become bf16 two at a time
-//   (v_cvt_scalef32_pk_bf16_fp8: a byte q is the E4M3 value q * 2^-9).
+//   32 clocks) three parts take 48 + 8 matrix clocks instead of 256 per 16x16
+//   outputs and 32 weights, and one packed fma forms two weight operands.
+//   (The quants as they are and the mins' share taken off afterwards is 3 to 5%
+//   faster, but channels of x far above the others at zero weights then leave
+//   errors of up to 10% of sum |w x|, where dequantised weights leave none.)
 //
 // An output that is not finite is computed again weight by weight in f32
 // (row_dot), so infinities, NaN and intermediate overflow come out as the
@@ -37,8 +39,8 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kGemmBufferWord3 = 0x00020000;  // raw 32-bit buffer, no swizzle
 constexpr uint32_t kHalf = 128;               // weights of half a super-block
@@ -47,59 +49,111 @@ constexpr uint32_t kSkip = 0x80000000u;       // buffer offset past every resour
 __device__ __forceinline__ u32x4 ld16(const uint8_t* p) {
   return *reinterpret_cast<const u32x4*>(p);
 }
-// Two of the four nibbles (one per byte of w, each 0..15) as bf16: byte q is
-// the FP8 E4M3 number q * 2^-9 (subnormal below 8), so the conversion scaled
-// by 2^9 gives q exactly.
-template <bool HIGH>
-__device__ __forceinline__ uint32_t nibbles_bf16(uint32_t w) {
-  return __builtin_bit_cast(uint32_t,
-                            __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 512.0f, HIGH));
-}
-// The 8 nibbles of a sub-block's two words (already masked to one per byte).
-__device__ __forceinline__ bf16x8 quants_bf16(uint32_t w0, uint32_t w1) {
-  return __builtin_bit_cast(bf16x8, u32x4{nibbles_bf16<false>(w0), nibbles_bf16<true>(w0),
-                                          nibbles_bf16<false>(w1), nibbles_bf16<true>(w1)});
+
+// The zero point of sub-block g of a weight row: the whole number of quant steps
+// nearest to its min, 0..15.  Every weight is then d*sc * (q - z) + rest with
+// |rest| at most the weight itself: q = z leaves the rest alone, another q is
+// at least half a step away, and where the min lies beyond the quants both terms
+// have one sign.  So the two sums a product is made of, over the first terms and
+// over the rests, are no larger than a few times sum |w x|, whatever the weights
+// and x.  (Sums over quants and mins apart are two large terms under a large x at
+// a small weight, whose roundings the difference keeps.)
+struct ZeroPoint {
+  uint32_t z;
+  float rest;  // d*sc*z - dmin*mn, rounded once (the products are exact)
+};
+__device__ __forceinline__ ZeroPoint zero_point(float d, float dmin, uint32_t sc, uint32_t mn) {
+  const float step = d * (float)sc, min = dmin * (float)mn;
+  // Any z gives the weights; NaN and infinities clamp.
+  const float z = rintf(__builtin_amdgcn_fmed3f(min * __builtin_amdgcn_rcpf(step), 0.f, 15.f));
+  return {(uint32_t)z, __builtin_fmaf(step, z, -min)};
 }
 
-// The upper halves of two registers: bf16(a) | bf16(b) << 16, truncated.
-__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+// A word or'ed over the four 16-lane rows.
+__device__ __forceinline__ uint32_t or_rows(uint32_t v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = a[0] | a[1];
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return b[0] | b[1];
 }
 
-// x = hi + mid + lo, three bf16 operands of eight values.
+// Operand scales of two sub-blocks, bytes 2p and 2p + 1 of sc (6-bit scales) and
+// z16 (zero points times 16): sc * 2^5 and z * sc * 2^-15.
+struct PairScale {
+  f16x2 s, zs;
+};
+__device__ __forceinline__ PairScale pair_scale(uint32_t sc, uint32_t z16, int p) {
+  // The half 0x6400 | b is 1024 + b, and the half b of one byte b * 2^-24.
+  const f16x2 up = {(_Float16)32.0f, (_Float16)32.0f};
+  const f16x2 off = {(_Float16)-32768.0f, (_Float16)-32768.0f};
+  const uint32_t b = __builtin_amdgcn_perm(0x64646464u, sc, p ? 0x04030402u : 0x04010400u);
+  const uint32_t z = __builtin_amdgcn_perm(0u, z16, p ? 0x0C030C02u : 0x0C010C00u);
+  const f16x2 s = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, b), up, off);
+  return {s, __builtin_bit_cast(f16x2, z) * s};
+}
+
+// Weight operand of one sub-block: the eight values sc * (q - z) * 2^-15, q the
+// high nibbles of w's bytes, whole numbers up to 945 and so exact.  The half
+// 16 q is the subnormal q * 2^-20, so one fma a pair forms them.
+__device__ __forceinline__ f16x8 weights_f16(u32x2 w, _Float16 s, _Float16 zs) {
+  const f16x2 ss = {s, s}, tt = {zs, zs};
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t h = __builtin_amdgcn_perm(0u, (i & 2 ? w.y : w.x) & 0xF0F0F0F0u,
+                                             i & 1 ? 0x0C030C02u : 0x0C010C00u);
+    o[i] = __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, h), ss, -tt));
+  }
+  return __builtin_bit_cast(f16x8, o);
+}
+constexpr float kOperandUp = 0x1p15f;  // takes the operands' 2^-15 off again
+
+// Scales x so that the largest of a row's block lies in [2^14, 2^15): up is
+// that power of two and down its inverse, both inside f32's normal range (an
+// infinity or NaN passes through unscaled or not and makes the row's outputs
+// so, which then take row_dot).
+struct BlockScale {
+  float up, down;
+};
+__device__ __forceinline__ BlockScale block_scale(float big) {
+  int e = (int)(__float_as_uint(big) >> 23) - 127;
+  e = max(-110, min(e, 127));
+  return {__uint_as_float((uint32_t)(127 + 14 - e) << 23),
+          __uint_as_float((uint32_t)(127 - 14 + e) << 23)};
+}
+
+// x = p[0] + 2^-11 p[1] + 2^-22 p[2], f16 operands of eight scaled values: each
+// part holds the next 11 bits, scaled up so that it keeps them as a normal
+// number.  Exact for values down to 2^-38 of the block's largest; below, off by
+// up to 2^-61 of it.
+constexpr float kPartUp = 0x1p11f, kPartDown = 0x1p-11f;
 struct Split3 {
-  bf16x8 hi, mid, lo;
+  f16x8 p[3];
 };
 __device__ __forceinline__ Split3 split3(const float (&x)[8]) {
 #pragma clang fp contract(off)
-  u32x4 h, m, l;
+  u32x4 o[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t a = __float_as_uint(x[2 * i]), b = __float_as_uint(x[2 * i + 1]);
-    const float ra = x[2 * i] - __uint_as_float(a & 0xFFFF0000u);
-    const float rb = x[2 * i + 1] - __uint_as_float(b & 0xFFFF0000u);
-    const uint32_t ma = __float_as_uint(ra), mb = __float_as_uint(rb);
-    const float la = ra - __uint_as_float(ma & 0xFFFF0000u);
-    const float lb = rb - __uint_as_float(mb & 0xFFFF0000u);
-    h[i] = pack_hi(a, b);
-    m[i] = pack_hi(ma, mb);
-    l[i] = pack_hi(__float_as_uint(la), __float_as_uint(lb));
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const f16x2 h = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(a, b));
+      o[c][i] = __builtin_bit_cast(uint32_t, h);
+      if (c == 2) break;
+      a = __builtin_fmaf((float)h.x, -kPartUp, a * kPartUp);  // exact
+      b = __builtin_fmaf((float)h.y, -kPartUp, b * kPartUp);
+    }
   }
-  return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m),
-          __builtin_bit_cast(bf16x8, l)};
+  return {{__builtin_bit_cast(f16x8, o[0]), __builtin_bit_cast(f16x8, o[1]),
+           __builtin_bit_cast(f16x8, o[2])}};
 }
 
 // The value is computed here: without this the compiler puts off the
 // additions of unrolled steps to their end and keeps every step's products in
 // registers until then.
 __device__ __forceinline__ void pin(floatx4& v) { asm volatile("" : "+v"(v)); }
-
-// The products of hi, and those of lo and mid, summed apart and then added.
-template <typename F>
-__device__ __forceinline__ floatx4 sum8(const Split3& x, F product) {
-  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  return product(x.hi, zero) + product(x.mid, product(x.lo, zero));
-}
 
 __device__ __forceinline__ bool is_finite(float v) {
   return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u;
@@ -135,7 +189,7 @@ __device__ __noinline__ float row_dot(const uint8_t* wrow, const float* x, const
 // share K, wave w taking half super-blocks w, w + WAVES, ... of 128 weights.
 // Per half super-block a wave loads its 16 x 128 x values once (lane (r, g):
 // row r, eight values of each of the four sub-blocks), splits them into the
-// three bf16 operands, and multiplies them with the NT tiles' weights (lane
+// three f16 operands, and multiplies them with the NT tiles' weights (lane
 // (r, g): weight row r, bytes 8g..8g+7 of each 32-byte run, whose low and
 // high nibbles are the operands of two sub-blocks).  The next half
 // super-block's x and weights are requested as soon as this one's registers
@@ -217,9 +271,6 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
   for (int i = 0; i < NT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   float ss[4] = {0.f, 0.f, 0.f, 0.f};
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  bf16x8 m8;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) m8[e] = (__bf16)-8.0f;
 
   // A wave's half super-blocks are all first halves or all second ones.
   static_assert(WAVES % 2 == 0, "half super-blocks alternate between the waves");
@@ -232,45 +283,51 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
   for (int i = 0; i < NT; ++i) load_w(i, hb);
   for (; hb < KH; hb += WAVES) {
     const uint32_t nx = hb + WAVES;
-    // Sub-block j of the half super-block: its x operands.
-    Split3 xs[4];
+    // Sub-block j's x: the row's largest, its sum, its operands.
+    float x[4][8], sx[4], big = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float x[8] = {xr[2 * j].x,     xr[2 * j].y,     xr[2 * j].z,     xr[2 * j].w,
-                    xr[2 * j + 1].x, xr[2 * j + 1].y, xr[2 * j + 1].z, xr[2 * j + 1].w};
+      const float t[8] = {xr[2 * j].x,     xr[2 * j].y,     xr[2 * j].z,     xr[2 * j].w,
+                          xr[2 * j + 1].x, xr[2 * j + 1].y, xr[2 * j + 1].z, xr[2 * j + 1].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[j][e] = t[e];
       if constexpr (NORM) {
         const float a[8] = {al[2 * j].x,     al[2 * j].y,     al[2 * j].z,     al[2 * j].w,
                             al[2 * j + 1].x, al[2 * j + 1].y, al[2 * j + 1].z, al[2 * j + 1].w};
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          ss[j] = __builtin_fmaf(x[e], x[e], ss[j]);
-          x[e] *= a[e];
+          ss[j] = __builtin_fmaf(x[j][e], x[j][e], ss[j]);
+          x[j][e] *= a[e];
         }
       }
-      xs[j] = split3(x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) big = fmaxf(big, fabsf(x[j][e]));
+      sx[j] = ((x[j][0] + x[j][1]) + (x[j][2] + x[j][3])) +
+              ((x[j][4] + x[j][5]) + (x[j][6] + x[j][7]));
     }
-    load_x(nx);
-    // -8 times the sub-block's sum of x, in both layouts: c8[j] where the
-    // tiles' accumulators want it (row 4g + e of every column), and sxg, what
-    // lane (r, g) supplies to the min product (row r, sub-block g).  The same
-    // products in the same order, so the two agree bit for bit.  The sum of
-    // the hi parts is exact but for the widest spreads of x, and mid and lo
-    // are added to it by one rounded addition: the matrix instruction
-    // truncates what it aligns below its largest term, which here, the mins
-    // having one sign, would add up over K (2.9e-7 from 64 bits at K = 4096
-    // with one chain of three, 1.7e-7 on the f32 matrix instructions).
-    floatx4 c8[4];
-    float sxg = 0.f;
+    const BlockScale bs = block_scale(max_xor32(max_xor16(big)));
+    Split3 xs[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      c8[j] = sum8(xs[j], [&](bf16x8 x, floatx4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, m8, c, 0, 0, 0);
-      });
-      const floatx4 t = sum8(xs[j], [&](bf16x8 x, floatx4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(m8, x, c, 0, 0, 0);
-      });
-      sxg = g == j ? t[0] : sxg;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[j][e] *= bs.up;
+      xs[j] = split3(x[j]);
     }
+    load_x(nx);
+    // What lane (r, g) supplies to the rests' product: row r's sum of sub-block
+    // g, the four lanes' shares added as they are dealt (the swap leaves sum j
+    // of one half of the lanes and sum j' of the other in the pair it returns).
+    const auto pair = [](auto r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+    const float s02 = pair(__builtin_amdgcn_permlane32_swap(
+        __float_as_uint(sx[0]), __float_as_uint(sx[2]), false, false));
+    const float s13 = pair(__builtin_amdgcn_permlane32_swap(
+        __float_as_uint(sx[1]), __float_as_uint(sx[3]), false, false));
+    const float sxg = pair(__builtin_amdgcn_permlane16_swap(
+        __float_as_uint(s02), __float_as_uint(s13), false, false));
+    // 2^k of row 4g + e, the accumulators' rows: four quarters of it, exactly.
+    const floatx4 down = __builtin_amdgcn_mfma_f32_16x16x4f32(0.25f * bs.down, 1.0f, zero, 0, 0, 0);
+    // x's own values are out of the registers by here (this instance would spill).
+    if constexpr (NT == 4 && NORM) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       // Scales and mins of the half's four sub-blocks, one per byte (the
@@ -279,36 +336,29 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_rows_kernel(const Q4kGemmParam
       const uint32_t mn4 =
           ((half ? hd[i].w >> 4 : hd[i].z) & mask_lo) | ((hd[i].z >> 2) & mask_hi);
       const float d = half_bits_to_float(hd[i].x), dmin = half_bits_to_float(hd[i].x >> 16);
-      // dmin*mn/8 - d*sc of sub-block g: what is left of the min after the
-      // quants' shift by 8, over -8.
-      const float mg = dmin * (float)((mn4 >> (8 * g)) & 0xFFu);
-      const float mng = __builtin_fmaf(mg, 0.125f, -(d * (float)((sc4 >> (8 * g)) & 0xFFu)));
-      bf16x8 wq[4];
-      wq[0] = quants_bf16(qa[i].x & 0x0F0F0F0Fu, qa[i].y & 0x0F0F0F0Fu);
-      wq[1] = quants_bf16((qa[i].x >> 4) & 0x0F0F0F0Fu, (qa[i].y >> 4) & 0x0F0F0F0Fu);
-      wq[2] = quants_bf16(qb[i].x & 0x0F0F0F0Fu, qb[i].y & 0x0F0F0F0Fu);
-      wq[3] = quants_bf16((qb[i].x >> 4) & 0x0F0F0F0Fu, (qb[i].y >> 4) & 0x0F0F0F0Fu);
+      const ZeroPoint zp = zero_point(d, dmin, (sc4 >> (8 * g)) & 0xFFu, (mn4 >> (8 * g)) & 0xFFu);
+      const uint32_t z4 = or_rows(zp.z << (8 * g + 4));
+      const PairScale s0 = pair_scale(sc4, z4, 0), s1 = pair_scale(sc4, z4, 1);
+      f16x8 wq[4];
+      wq[0] = weights_f16(u32x2{qa[i].x << 4, qa[i].y << 4}, s0.s.x, s0.zs.x);
+      wq[1] = weights_f16(qa[i], s0.s.y, s0.zs.y);
+      wq[2] = weights_f16(u32x2{qb[i].x << 4, qb[i].y << 4}, s1.s.x, s1.zs.x);
+      wq[3] = weights_f16(qb[i], s1.s.y, s1.zs.y);
       load_w(i, nx);
-      floatx4 s[4];
+      // The parts are summed apart and then added, this step's share by itself:
+      // one rounding at the size of the running total per step.
+      floatx4 t[3] = {zero, zero, zero};
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xs[j].hi, wq[j], c8[j], 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xs[j].mid, wq[j], s[j], 0, 0, 0);
+        for (int c = 0; c < 3; ++c)
+          t[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[j].p[c], wq[j], t[c], 0, 0, 0);
+      const floatx4 m = __builtin_amdgcn_mfma_f32_16x16x4f32(sxg, zp.rest, zero, 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xs[j].lo, wq[j], s[j], 0, 0, 0);
-      // This step's share is summed by itself: one rounding at the size of
-      // the running total per step.
-      floatx4 t = __builtin_amdgcn_mfma_f32_16x16x4f32(sxg, mng, zero, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float d1 = d * (float)((sc4 >> (8 * j)) & 0xFFu);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(s[j][e], d1, t[e]);
+      for (int e = 0; e < 4; ++e) {
+        const float u = __builtin_fmaf(__builtin_fmaf(t[2][e], kPartDown, t[1][e]), kPartDown, t[0][e]);
+        acc[i][e] += __builtin_fmaf(u * (kOperandUp * d), down[e], m[e]);
       }
-      acc[i] += t;
       pin(acc[i]);  // one tile's operands at a time in registers
     }
   }
@@ -642,9 +692,6 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p, cons
   }
 }
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
 // Many rows.  Here the matrix core's share is large enough for the scaling of
 // every sub-block's sum in f32 (four additions a tile and lane) to cost more
 // than it, so the 6-bit scales go into the weight operand: sc*(q - 8) is a
@@ -775,7 +822,7 @@ __device__ __forceinline__ void lds_barrier() {
 // Weight operand of one sub-block: the eight values sc*(q - 8), q the high
 // nibbles of w's bytes.  The half 0x5400 | 16 q is 64 + q, so one fma per pair,
 // (64 + q) sc - 72 sc, gives it exactly (72 sc = 9 sc * 8 fits 11 bits).
-__device__ __forceinline__ f16x8 weights_f16(u32x2 w, _Float16 sc, _Float16 sc72) {
+__device__ __forceinline__ f16x8 weights8_f16(u32x2 w, _Float16 sc, _Float16 sc72) {
   const f16x2 s = {sc, sc}, t = {sc72, sc72};
   u32x4 o;
 #pragma unroll
@@ -923,7 +970,7 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
           const _Float16 sch = __builtin_bit_cast(_Float16, (unsigned short)(0x6400u | byte)) -
                                (_Float16)1024.0f;
           const u32x2 w = j ? q[i] : u32x2{q[i].x << 4, q[i].y << 4};
-          wq[i] = weights_f16(w, sch, sch * (_Float16)72.0f);
+          wq[i] = weights8_f16(w, sch, sch * (_Float16)72.0f);
         }
       };
       f16x8 xs[4][kParts], wq[2][2];

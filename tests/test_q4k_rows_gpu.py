@@ -272,7 +272,9 @@ def near_zero_blocks(seed, N, K, cols):
     return blk.reshape(-1)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 515, 1024), (2, 301, 2304), (1, 130, 4096)])
+# One and two rows; a few rows.
+@pytest.mark.parametrize("M,N,K", [(1, 515, 1024), (2, 301, 2304), (1, 130, 4096), (5, 200, 512),
+                                   (13, 700, 2816), (40, 130, 5120)])
 def test_small_weights_under_large_x(gpu, M, N, K):
     """Channels of x up to 1e12 times the others at weights that are zero or
     nearly: each output is within 2e-6 of sum |w x|, 33 roundings of f32 at that
