@@ -424,7 +424,8 @@ int sts_debug_set_wait_limit(uint32_t polls);
  * reference's [B, 1, K] input), y [batch][n], residual [batch][n] or NULL.
  * k must be a multiple of 256 and at most 16384; weights and x 16-byte
  * aligned.  From 4 rows on (8 where n < 2048) the rows share the weights as
- * in sts_q4k_gemm, whose order of summation then applies.
+ * in sts_q4k_gemm, whose order of summation and use of library memory then
+ * apply: a row's last bits depend on the size of its batch.
  */
 int sts_q4k_matvec(const uint8_t* weights, const float* x, const float* residual, float* y,
                    uint32_t batch, uint32_t k, uint32_t n, void* stream);
@@ -448,10 +449,14 @@ int sts_q4k_dequant(const uint8_t* weights, float* out, uint32_t k, uint32_t n, 
  * product for more than one row, which the reference runs with the
  * one-thread-per-output shader (q4k_matmul with M > 1, gguf.rs:810-897 and
  * wgsl/shader_q4k.wgsl; q4k_matmul_with_residual, gguf.rs:899-905).  The
- * products run on the bf16 matrix cores with every f32 x as the exact sum of
- * three bf16 values and the quants as they are, accumulated and scaled in
- * f32: no operand is rounded, and the result is as close to the exact product
- * as with f32 matrix instructions on the dequantised weights.  With
+ * products run on the f16 matrix cores and accumulate in f32: x as the sum of
+ * three f16 values, scaled per row and 128 columns (exact down to 2^-38 of the
+ * block's largest value; one or two rows in f32 throughout), the weights as
+ * whole quant steps and a remainder no larger than the weight, rounded once.  The
+ * result is as close to the exact product as with f32 matrix instructions on the
+ * dequantised weights, also where a channel of x is far larger than the others.
+ * Large products (see below) round x to 23 bits instead of 24, down to 2^-39 of
+ * the largest value in its 256 columns.  With
  * swiglu != 0 the matrix has n = 2F rows and
  * y[m][j] = silu(G[m][j]) * G[m][j + F] for j < F (the SwiGLU of
  * wgsl/shader_swiglu.wgsl applied to the product; residual must be NULL).
@@ -461,9 +466,9 @@ int sts_q4k_dequant(const uint8_t* weights, float* out, uint32_t k, uint32_t n, 
  * fused; its sum of squares is taken in this kernel's order, not the
  * shader's).  k must be a multiple of 256 in 256..16384; above 4096 (the
  * temporal FFN's linear_out, k = 11264) without norm_alpha or swiglu.
- * Large products (from 33 rows) keep x's operands in the stream's library
- * workspace (at most 1024 rows' at a time); where that would have to grow while
- * the stream is being captured, the call runs without it.
+ * Large products (from 33 rows and 1.5e9 multiplications, without norm_alpha
+ * and swiglu) keep x's operands in library memory, at most 1024 rows' at a time
+ * (see the rules above: not while the stream is being captured).
  * x rows, norm_alpha and weights 16-byte aligned; ldx, ldy, ldr are row
  * strides in floats (ldx a multiple of 4).
  */

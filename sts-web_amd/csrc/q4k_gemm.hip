@@ -11,8 +11,7 @@
 //   v_mfma_f32_16x16x32_f16 on x's parts, each with an accumulator of its own,
 //   give sum sc*(q - z)*x with exact products and f32 accumulation; d scales that
 //   sum in f32, and rest_j times the sub-block's sum of x is added by one
-//   v_mfma_f32_16x16x4f32 per four sub-blocks.  (Products of many rows still take
-//   z = 8 throughout, see there.)
+//   v_mfma_f32_16x16x4f32 per four sub-blocks.
 //   Against v_mfma_f32_16x16x4f32 on dequantised weights (one per 4 weights,
 //   32 clocks) three parts take 48 + 8 matrix clocks instead of 256 per 16x16
 //   outputs and 32 weights, and one packed fma forms two weight operands.
@@ -692,45 +691,53 @@ __global__ __launch_bounds__(64) void q4k_vec_kernel(const Q4kGemmParams p, cons
   }
 }
 
-// Many rows.  Here the matrix core's share is large enough for the scaling of
-// every sub-block's sum in f32 (four additions a tile and lane) to cost more
-// than it, so the 6-bit scales go into the weight operand: sc*(q - 8) is a
-// whole number up to 504, exact in f16, and d alone is left for the super-block's
-// sum.  x then has to be f16 too: the 256 values of a row and super-block are
-// scaled by a power of two that brings the largest to 2^14..2^15 and split
-// into kParts f16 values, each the rest rounded to nearest (two parts hold 22
-// bits and the sign of the rest, three all 24, both down to 2^-39 of the
-// largest).  The mins, (dmin*mn - 8*d*sc) times the sub-block's sum of x, go
-// through v_mfma_f32_16x16x4f32 as in q4k_rows_kernel.
+// Many rows.  x as two f16 parts, the first rounded to nearest and the second
+// what it leaves: 23 bits of every value down to 2^-28 of the largest in its row
+// and super-block.  The f32 sums round at 24 bits of the running total, over
+// which this is not seen (x Gaussian, K = 4096: 1.2e-7 from 64 bits, with all 24
+// bits on the f32 matrix instructions 1.7e-7).  Super-blocks of 16 rows that
+// hold smaller values (beside an outlier) get a third part, whose products only
+// they pay for: then 23 bits down to 2^-39.
 constexpr int kParts = 2;
 constexpr int kTileM = 64, kTileN = 128;
 
 // What split_planes_kernel writes for `rows` rows (a multiple of 64) of K
 // columns, in floats: operand units of 64 x 16 bytes per (16-row tile mt,
 // sub-block kb, part), entry g*16 + r being row r, columns 8g..8g+7, as lane
-// (r, g) of a matrix instruction wants it; the sums of x per (mt, kb, row);
-// and the inverse scales per (mt, super-block, row).
+// (r, g) of a matrix instruction wants it; the third parts' units in the same
+// order, written only where they are used; the sums of x per (mt, kb, row); and
+// the scales per (mt, super-block, row), negated where there is a third part.
 struct TilePlanes {
   u32x4* units;
+  u32x4* third;
   float* sums;
   float* scales;
   static size_t floats(size_t rows, size_t KB) {
-    return rows / 16 * KB * kParts * 256 + rows * KB + rows * (KB / 8);
+    return rows / 16 * KB * (kParts + 1) * 256 + rows * KB + rows * (KB / 8);
   }
   TilePlanes(float* p, size_t rows, size_t KB)
       : units(reinterpret_cast<u32x4*>(p)),
-        sums(p + rows / 16 * KB * kParts * 256),
+        third(units + rows / 16 * KB * kParts * 64),
+        sums(p + rows / 16 * KB * (kParts + 1) * 256),
         scales(sums + rows * KB) {}
 };
+
+// Element i of the parts of the scaled value y; returns what they leave, times
+// 2^11 (exact).
+__device__ __forceinline__ float split_parts(float y, f16x8 (&h)[kParts], int i) {
+  static_assert(kParts == 2, "two parts");
+  h[0][i] = (_Float16)y;
+  const float rest = __builtin_fmaf((float)h[0][i], -kPartUp, y * kPartUp);
+  h[1][i] = (_Float16)rest;
+  return rest - (float)h[1][i];
+}
 
 // One wave per 16-row tile and super-block: lane (r, g) takes row r, columns
 // 8g..8g+7 of each of the eight sub-blocks.  Rows past M become zeros.  The
 // sums of x are taken in f64 and rounded once.
 __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restrict__ x,
-                                                           uint64_t ldx, uint32_t M, uint32_t SB,
-                                                           u32x4* __restrict__ units,
-                                                           float* __restrict__ sums,
-                                                           float* __restrict__ scales) {
+                                                              uint64_t ldx, uint32_t M,
+                                                              uint32_t SB, const TilePlanes out) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
@@ -740,6 +747,7 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restri
   const float* row = x + (size_t)(m < M ? m : 0) * ldx + 256 * (size_t)sb + 8 * g;
   float v[8][8];
   float big = 0.f;
+  uint32_t least = ~0u;  // twice the bits of the smallest magnitude but zero, less one
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float4 a = *reinterpret_cast<const float4*>(row + 32 * j);
@@ -749,41 +757,42 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restri
     for (int e = 0; e < 8; ++e) {
       v[j][e] = m < M ? t[e] : 0.f;
       big = fmaxf(big, fabsf(v[j][e]));
+      least = min(least, 2 * __float_as_uint(v[j][e]) - 1);
     }
   }
   big = max_xor32(max_xor16(big));
-  // 2^(14 - e) for the largest value's exponent e, inside f32's normal range
-  // (an infinity or NaN passes through unscaled or not and makes the row's
-  // outputs so, which then take row_dot).
-  int e = (int)(__float_as_uint(big) >> 23) - 127;
-  e = max(-110, min(e, 127));
-  const float up = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
-  if (g == 0)
-    scales[((size_t)mt * SB + sb) * 16 + r] = __uint_as_float((uint32_t)(127 - 14 + e) << 23);
+  const BlockScale bs = block_scale(big);
+  // Of values below 2^-27 of the largest's power of two, two parts can leave more
+  // than 2^-23.
+  const uint32_t exponent = __float_as_uint(big) >> 23;
+  const bool third = __any(least < (exponent > 27 ? exponent - 27 : 0u) << 24);
+  if (g == 0) out.scales[((size_t)mt * SB + sb) * 16 + r] = third ? -bs.down : bs.down;
+  const size_t kb0 = (size_t)mt * SB * 8 + 8 * sb;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const size_t kb = (size_t)mt * SB * 8 + 8 * sb + j;
-    u32x4* u = units + kb * kParts * 64 + (g * 16 + r);
-    float rest[8];
+    u32x4* u = out.units + (kb0 + j) * kParts * 64 + (g * 16 + r);
     double q = 0.0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      rest[i] = v[j][i] * up;
-      q += (double)v[j][i];
-    }
+    for (int i = 0; i < 8; ++i) q += (double)v[j][i];
+    f16x8 h[kParts];
 #pragma unroll
-    for (int c = 0; c < kParts; ++c) {
-      f16x8 h;
+    for (int i = 0; i < 8; ++i) split_parts(v[j][i] * bs.up, h, i);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        h[i] = (_Float16)rest[i];
-        rest[i] -= (float)h[i];
-      }
-      u[64 * c] = __builtin_bit_cast(u32x4, h);
-    }
+    for (int c = 0; c < kParts; ++c) u[64 * c] = __builtin_bit_cast(u32x4, h[c]);
     q += __shfl_xor(q, 16, 64);
     q += __shfl_xor(q, 32, 64);
-    if (g == 0) sums[kb * 16 + r] = (float)q;
+    if (g == 0) out.sums[(kb0 + j) * 16 + r] = (float)q;
+  }
+  if (!third) return;
+  // Rare: x is read again (the compiler not knowing that it is) rather than kept.
+  asm volatile("" : "+v"(row));
+#pragma nounroll
+  for (int j = 0; j < 8; ++j) {
+    f16x8 h[kParts], rest;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      rest[i] = (_Float16)(split_parts((m < M ? row[32 * j + i] : 0.f) * bs.up, h, i) * kPartUp);
+    out.third[(kb0 + j) * 64 + (g * 16 + r)] = __builtin_bit_cast(u32x4, rest);
   }
 }
 
@@ -794,13 +803,13 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restri
 // LDS through registers, two buffers each: a step's x operands
 // one step ahead, a super-block's weight bytes
 // (128 x 144) come in two batches during the super-block before.  The
-// super-block's products accumulate in the matrix core, those of
-// the first part and of the others apart (the others' sums are small, so that
-// only the first part's eight additions round at the size of the result); then
+// super-block's products accumulate in the matrix core, each part's apart (only
+// the first part's eight additions round at the size of the result); then
 // they are scaled by d and the row's scale and added to the total.
 struct Q4kTileParams {
   const uint8_t* w;
   const u32x4* units;
+  const u32x4* third;
   const float* sums;
   const float* scales;
   const float* x;  // the rows themselves, for outputs that are not finite
@@ -819,20 +828,23 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Weight operand of one sub-block: the eight values sc*(q - 8), q the high
-// nibbles of w's bytes.  The half 0x5400 | 16 q is 64 + q, so one fma per pair,
-// (64 + q) sc - 72 sc, gives it exactly (72 sc = 9 sc * 8 fits 11 bits).
-__device__ __forceinline__ f16x8 weights8_f16(u32x2 w, _Float16 sc, _Float16 sc72) {
-  const f16x2 s = {sc, sc}, t = {sc72, sc72};
-  u32x4 o;
+// A weight row's super-block header as lane (r, g) uses it: the eight scales and
+// zero points, one per byte, d, and the rests of sub-blocks g and 4 + g.
+__device__ __forceinline__ void tile_header(u32x4 h, int g, uint32_t (&sc)[2], uint32_t (&zp)[2],
+                                            float& d, float (&rest)[2]) {
+  sc[0] = h.y & 0x3F3F3F3Fu;
+  sc[1] = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+  const uint32_t mn[2] = {h.z & 0x3F3F3F3Fu,
+                          ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u)};
+  d = half_bits_to_float(h.x);
+  const float dmin = half_bits_to_float(h.x >> 16);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t h = __builtin_amdgcn_perm(0x54545454u, (i & 2 ? w.y : w.x) & 0xF0F0F0F0u,
-                                             i & 1 ? 0x04030402u : 0x04010400u);
-    o[i] = __builtin_bit_cast(
-        uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, h), s, -t));
+  for (int hf = 0; hf < 2; ++hf) {
+    const ZeroPoint z =
+        zero_point(d, dmin, (sc[hf] >> (8 * g)) & 0xFFu, (mn[hf] >> (8 * g)) & 0xFFu);
+    zp[hf] = or_rows(z.z << (8 * g + 4));
+    rest[hf] = z.rest;
   }
-  return __builtin_bit_cast(f16x8, o);
 }
 
 __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p) {
@@ -856,10 +868,18 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
 
   // x: wave w stages 16-row tile w, contiguous in memory and in LDS.
   constexpr int XU = 2 * kParts;
-  const u32x4* xsrc = p.units + (size_t)(mb * 4 + wave) * KB * kParts * 64 + lane;
+  // (Buffer resources leave the addresses to scalar registers; none is larger
+  // than 4 MiB.)
+  auto rsrc = [](const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes,
+                                             kGemmBufferWord3);
+  };
+  const __amdgpu_buffer_rsrc_t xrs =
+      rsrc(p.units + (size_t)(mb * 4 + wave) * KB * kParts * 64, KB * kParts * 1024);
   auto load_x = [&](u32x4 (&d)[XU], uint32_t s) {
 #pragma unroll
-    for (int u = 0; u < XU; ++u) d[u] = xsrc[(size_t)s * (XU * 64) + 64 * u];
+    for (int u = 0; u < XU; ++u)
+      d[u] = __builtin_amdgcn_raw_buffer_load_b128(xrs, lane * 16, (s * XU + u) * 1024, 0);
   };
   auto put_x = [&](int b, const u32x4 (&d)[XU]) {
 #pragma unroll
@@ -867,40 +887,54 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
   };
   // Weights: 1152 entries of 16 bytes, entry i being bytes 16 (i % 9) .. of
   // weight row i / 9; thread t moves entries t, t + 256, ..., the last half
-  // round entry 1151 once more.  Rows past the last re-read it.
+  // round entry 1151 once more.  Rows past the last read zeros.
   constexpr int WE = kTileN * 9, WU = (WE + 255) / 256;
   uint32_t wsrc[WU], wdst[WU];
   const uint32_t nfirst = nb * kTileN;
 #pragma unroll
   for (int k = 0; k < WU; ++k) {
     wdst[k] = min((uint32_t)tid + 256 * k, (uint32_t)WE - 1);
-    wsrc[k] = (min(nfirst + wdst[k] / 9, p.N - 1) - nfirst) * (uint32_t)row_bytes + 16 * (wdst[k] % 9);
+    wsrc[k] = wdst[k] / 9 * (uint32_t)row_bytes + 16 * (wdst[k] % 9);
   }
-  const uint8_t* wrow0 = p.w + (size_t)nfirst * row_bytes;
+  const __amdgpu_buffer_rsrc_t wrs =
+      rsrc(p.w + (size_t)nfirst * row_bytes, min((uint32_t)kTileN, p.N - nfirst) * (uint32_t)row_bytes);
   // In two batches, entries 0-1 and 2-4 of each thread.
   auto load_w = [&](u32x4 (&d)[3], int batch, uint32_t sb) {
-    const uint8_t* src = wrow0 + (size_t)sb * kQ4kBlockBytes;
 #pragma unroll
-    for (int k = 0; k < 2 + batch; ++k) d[k] = ld16(src + wsrc[2 * batch + k]);
+    for (int k = 0; k < 2 + batch; ++k)
+      d[k] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wsrc[2 * batch + k], sb * kQ4kBlockBytes, 0);
   };
   auto put_w = [&](uint32_t b, const u32x4 (&d)[3], int batch) {
 #pragma unroll
     for (int k = 0; k < 2 + batch; ++k) wb[b][wdst[2 * batch + k]] = d[k];
   };
+  // Third parts of the four row tiles (at most 2 MiB).
+  const __amdgpu_buffer_rsrc_t x3rs = rsrc(p.third + (size_t)mb * 4 * KB * 64, 4 * KB * 1024);
   // Per super-block: row sums for the min product (row r of tile t, sub-block
   // g of each half) and the inverse scales of rows 4g .. 4g+3.
-  const float* sxsrc = p.sums + (size_t)mb * 4 * KB * 16 + g * 16 + r;
-  const float* scsrc = p.scales + (size_t)mb * 4 * SB * 16 + 4 * g;
+  const __amdgpu_buffer_rsrc_t sxrs = rsrc(p.sums + (size_t)mb * 4 * KB * 16, 4 * KB * 64);
+  const __amdgpu_buffer_rsrc_t scrs = rsrc(p.scales + (size_t)mb * 4 * SB * 16, 4 * SB * 64);
   auto load_sx = [&](float (&d)[4][2], uint32_t sb) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) d[t][hf] = sxsrc[((size_t)t * KB + 8 * sb + 4 * hf) * 16];
+      for (int hf = 0; hf < 2; ++hf)
+        d[t][hf] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(sxrs, lane * 4,
+                                                        (t * KB + 8 * sb + 4 * hf) * 64, 0));
   };
   auto load_scale = [&](floatx4 (&d)[4], uint32_t sb) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-      d[t] = *reinterpret_cast<const floatx4*>(scsrc + ((size_t)t * SB + sb) * 16);
+      d[t] = __builtin_bit_cast(
+          floatx4, __builtin_amdgcn_raw_buffer_load_b128(scrs, 16 * g, (t * SB + sb) * 64, 0));
+  };
+  // Lanes 0..3: a negative value where row tile `lane` has third parts (the
+  // others read past the resource: zeros).
+  auto load_flags = [&](uint32_t sb) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(scrs, lane < 4 ? lane * SB * 64 : kSkip,
+                                                    sb * 64, 0));
   };
 
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -920,38 +954,58 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
   load_w(wr, 1, sb0);
   put_w(0, wr, 1);
   put_x(0, xr);
+  float flags = load_flags(sb0);
   lds_barrier();
   for (uint32_t sb = sb0; sb < sb1; ++sb) {
     const uint32_t wcur = (sb - sb0) & 1;
     const u32x4* wt = &wb[wcur][(wave * 32 + r) * 9];
     floatx4 part[4][2], rest[4][2];
-    // Scales, one per byte (sub-blocks 0-3, 4-7), and 8*d*sc - dmin*mn of
-    // sub-blocks g and 4 + g.
-    uint32_t sc[2][2];
+    // Scales and zero points, one per byte (sub-blocks 0-3, 4-7), and the rests
+    // of sub-blocks g and 4 + g.
+    uint32_t sc[2][2], zp[2][2];
     float d[2], mc[2][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const u32x4 h = wt[16 * 9 * i];
-      sc[i][0] = h.y & 0x3F3F3F3Fu;
-      sc[i][1] = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-      const uint32_t mn0 = h.z & 0x3F3F3F3Fu;
-      const uint32_t mn1 = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-      d[i] = half_bits_to_float(h.x);
-      const float dmin = half_bits_to_float(h.x >> 16);
-      const float d8 = 8.0f * d[i];
-      mc[i][0] = __builtin_fmaf(d8, (float)((sc[i][0] >> (8 * g)) & 0xFFu),
-                                -(dmin * (float)((mn0 >> (8 * g)) & 0xFFu)));
-      mc[i][1] = __builtin_fmaf(d8, (float)((sc[i][1] >> (8 * g)) & 0xFFu),
-                                -(dmin * (float)((mn1 >> (8 * g)) & 0xFFu)));
-    }
+    for (int i = 0; i < 2; ++i) tile_header(wt[16 * 9 * i], g, sc[i], zp[i], d[i], mc[i]);
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       // Step s: its operands are in buffers it & 1.
       const uint32_t s = 4 * sb + it;
       const int b = it & 1;
       load_x(xr, min(s + 1, slast));
+      // The third parts' products, of the row tiles that have them, between two
+      // steps: the scheduler has no overlap to lose there.
+      const uint32_t third = it == 1 ? (uint32_t)__ballot(flags < 0.f) : 0u;
+      if (it == 1 && third) {
+#pragma nounroll
+        for (int k = 0; k < 8; ++k) {
+          f16x8 w[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const u32x2 q = reinterpret_cast<const u32x2*>(wt + 16 * 9 * i + 1 + (k & 6))[g];
+            const PairScale ps = pair_scale(sc[i][k >> 2] >> (8 * (k & 3)),
+                                            zp[i][k >> 2] >> (8 * (k & 3)), 0);
+            const uint32_t sh = k & 1 ? 0u : 4u;
+            w[i] = weights_f16(u32x2{q.x << sh, q.y << sh}, ps.s.x, ps.zs.x);
+          }
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            if (!(third >> t & 1u)) continue;
+            const f16x8 x3 = __builtin_bit_cast(
+                f16x8, __builtin_amdgcn_raw_buffer_load_b128(x3rs, lane * 16,
+                                                             (t * KB + 8 * sb + k) * 1024, 0));
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const floatx4 u = __builtin_amdgcn_mfma_f32_16x16x32_f16(x3, w[i], zero, 0, 0, 0);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                rest[t][i][e] = __builtin_fmaf(u[e], kPartDown, rest[t][i][e]);
+            }
+          }
+        }
+      }
       if (it == 0) load_w(wr, 0, min(sb + 1, sb1 - 1));
       if (it == 2) load_w(wr, 1, min(sb + 1, sb1 - 1));
+      if (it == 2) flags = load_flags(min(sb + 1, sb1 - 1));
       if (it == 3) {
         load_sx(sx, sb);
         load_scale(xsc, sb);
@@ -960,20 +1014,13 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         q[i] = reinterpret_cast<const u32x2*>(wt + 16 * 9 * i + 1 + 2 * it)[g];
-      // Weight tile i's operands for sub-block j.
-      auto weights = [&](f16x8 (&wq)[2], int j) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int k = 2 * it + j;
-          // sc as f16: the half 0x6400 | sc is 1024 + sc.
-          const uint32_t byte = (sc[i][k >> 2] >> (8 * (k & 3))) & 0xFFu;
-          const _Float16 sch = __builtin_bit_cast(_Float16, (unsigned short)(0x6400u | byte)) -
-                               (_Float16)1024.0f;
-          const u32x2 w = j ? q[i] : u32x2{q[i].x << 4, q[i].y << 4};
-          wq[i] = weights8_f16(w, sch, sch * (_Float16)72.0f);
-        }
-      };
+      // Weight tile i's operands for the step's two sub-blocks.
       f16x8 xs[4][kParts], wq[2][2];
+      auto weights = [&](int i) {
+        const PairScale ps = pair_scale(sc[i][it >> 1], zp[i][it >> 1], it & 1);
+        wq[0][i] = weights_f16(u32x2{q[i].x << 4, q[i].y << 4}, ps.s.x, ps.zs.x);
+        wq[1][i] = weights_f16(q[i], ps.s.y, ps.zs.y);
+      };
       auto read_x = [&](int t, int j) {
 #pragma unroll
         for (int c = 0; c < kParts; ++c)
@@ -981,8 +1028,8 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
       };
 #pragma unroll
       for (int t = 0; t < 4; ++t) read_x(t, 0);
-      weights(wq[0], 0);
-      weights(wq[1], 1);
+      weights(0);
+      weights(1);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -1015,8 +1062,10 @@ __global__ __launch_bounds__(256, 2) void q4k_tile_kernel(const Q4kTileParams p)
         floatx4 m = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[t][0], mc[i][0], zero, 0, 0, 0);
         m = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[t][1], mc[i][1], m, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          acc[t][i][e] += __builtin_fmaf(part[t][i][e] + rest[t][i][e], d[i] * xsc[t][e], m[e]);
+        for (int e = 0; e < 4; ++e) {
+          const float u = __builtin_fmaf(rest[t][i][e], kPartDown, part[t][i][e]);
+          acc[t][i][e] += __builtin_fmaf(u * (kOperandUp * d[i]), fabsf(xsc[t][e]), m[e]);
+        }
         pin(acc[t][i]);
       }
   }
@@ -1109,6 +1158,7 @@ int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
     Q4kTileParams t;
     t.w = p.w[0];
     t.units = planes.units;
+    t.third = planes.third;
     t.sums = planes.sums;
     t.scales = planes.scales;
     t.x = p.x + (size_t)m0 * p.ldx;
@@ -1124,7 +1174,7 @@ int launch_tiles(const Q4kGemmParams& p, hipStream_t stream, bool* done) {
     t.mtiles = (t.M + kTileM - 1) / kTileM;
     t.ksplit = ksplit;
     hipLaunchKernelGGL(split_planes_kernel, dim3((SB + 3) / 4, t.mtiles * 4), dim3(256), 0, stream,
-                       t.x, t.ldx, t.M, SB, planes.units, planes.sums, planes.scales);
+                       t.x, t.ldx, t.M, SB, planes);
     STS_HIP(hipGetLastError());
     const uint64_t grid = (uint64_t)((nblocks * ksplit + 7) / 8) * 8 * t.mtiles;
     if (grid > 0x7FFFFFFFull) return fail(STS_ERR_INVALID, "GEMM N = %u too large", p.N);

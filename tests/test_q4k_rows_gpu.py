@@ -132,6 +132,11 @@ def test_tiles_edges(gpu, M, N, K, res):
     ref = (xd @ wt.T.contiguous()).cpu().numpy() + (r.astype(np.float64) if res else 0.0)
     tol = 1e-5 * q4k_bound(blocks, x, N) + (1e-6 * np.abs(r) if res else 0.0)
     assert (np.abs(got - ref) <= tol).all(), (np.abs(got - ref) / tol).max()
+    # Row by row, the residual's own rounding aside.
+    d, own = got - ref, ref - (r.astype(np.float64) if res else 0.0)
+    off, norm = np.linalg.norm(d, axis=1), np.linalg.norm(own, axis=1)
+    print(f"  worst row {(off / norm).max():.2e}", flush=True)
+    assert (off <= 3e-7 * norm + (2.0 ** -24 * np.linalg.norm(got, axis=1) if res else 0.0)).all()
     again = host(sts_attn.q4k_gemm(dev(x), w, residual=dev(r) if res else None))
     np.testing.assert_array_equal(again, got)
 
@@ -159,6 +164,8 @@ def test_tiles_captured_without_workspace(gpu):
         assert (np.abs(host(out) - ref) <= tol).all()
         eager = host(sts_attn.q4k_gemm(xd, w))
         assert (np.abs(eager - ref) <= tol).all()
+        for y in (host(out), eager):
+            assert (np.linalg.norm(y - ref, axis=1) <= 3e-7 * np.linalg.norm(ref, axis=1)).all()
 
 
 @pytest.mark.parametrize("N,K,B,res", [(4096, 1024, 3, True), (4096, 1024, 4, True),
@@ -272,9 +279,10 @@ def near_zero_blocks(seed, N, K, cols):
     return blk.reshape(-1)
 
 
-# One and two rows; a few rows.
+# One and two rows; a few rows; the tiles of many rows (the last two).
 @pytest.mark.parametrize("M,N,K", [(1, 515, 1024), (2, 301, 2304), (1, 130, 4096), (5, 200, 512),
-                                   (13, 700, 2816), (40, 130, 5120)])
+                                   (13, 700, 2816), (40, 130, 5120), (64, 11265, 2304),
+                                   (130, 41001, 512)])
 def test_small_weights_under_large_x(gpu, M, N, K):
     """Channels of x up to 1e12 times the others at weights that are zero or
     nearly: each output is within 2e-6 of sum |w x|, 33 roundings of f32 at that
