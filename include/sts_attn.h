@@ -566,8 +566,8 @@ int sts_depformer_destroy(sts_depformer* d);
  * rand [batch][num_steps], penalty_tokens [batch][num_steps][30],
  * num_penalty [batch][num_steps] -> tokens [batch][num_steps]; optional
  * logits [num_steps][batch][out_vocab] receives each step's logits before
- * sampling.  All device pointers; nothing is read back, so the call can be
- * captured in a HIP graph.  The KV caches start empty every call (the
+ * sampling.  All device pointers; nothing is allocated or read back, so the call
+ * can be captured in a HIP graph.  The KV caches start empty every call (the
  * reference clears them per frame, depth_engine.rs:1497-1509).
  */
 int sts_depformer_generate(sts_depformer* d, const float* temporal_hidden,

@@ -32,6 +32,7 @@ struct Q4kGemmParams {
   // the row's 1/rms to its outputs.
   const float* norm_alpha = nullptr;
   float norm_eps = 0.f;
+  bool scratch = true;  // may use library memory (many rows)
 };
 // K above 4096 takes no RMSNorm or SwiGLU and Z = 1 only.  (q4k_gemm.hip)
 int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream);

@@ -224,6 +224,7 @@ int sts_depformer_generate(sts_depformer* d, const float* temporal_hidden,
   ip.M = batch;
   ip.N = D;
   ip.K = c.temporal_dim;
+  ip.scratch = false;  // generate allocates nothing, whatever the batch
   if (int rc = sts::launch_q4k_gemm(ip, st)) return rc;
 
   auto gemm = [&](const uint8_t* w, const float* x, uint32_t K, uint32_t N, const float* res,
@@ -242,6 +243,7 @@ int sts_depformer_generate(sts_depformer* d, const float* temporal_hidden,
     p.N = N;
     p.K = K;
     p.swiglu_f = swiglu_f;
+    p.scratch = false;
     return sts::launch_q4k_gemm(p, st);
   };
 

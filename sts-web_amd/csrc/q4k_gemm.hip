@@ -1262,8 +1262,8 @@ int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   // launches (x split, K ranges summed): 48 rows x [12288, 4096] 37 against
   // 50 us here, 112 x [4096, 4096] 33 against 51, but 80 x [4096, 4096] 32.5
   // against 29.8, 32 x [12288, 4096] 34.6 against 29.7.
-  if (p.M > 32 && (uint64_t)mtiles * 16 * p.N * p.K >= 1500000000ull && p.Z == 1 && !p.swiglu_f &&
-      !p.norm_alpha) {
+  if (p.scratch && p.M > 32 && (uint64_t)mtiles * 16 * p.N * p.K >= 1500000000ull && p.Z == 1 &&
+      !p.swiglu_f && !p.norm_alpha) {
     bool done = false;
     if (int rc = launch_tiles(p, stream, &done)) return rc;
     if (done) return STS_OK;

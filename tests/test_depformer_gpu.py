@@ -18,6 +18,7 @@ import torch
 import oracle
 import sts_attn
 from test_oracle_depformer import CFG
+from test_workspace_gpu import _stream_pool, fresh_stream  # noqa: F401 (fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -438,6 +439,46 @@ def test_depformer_few_streams_as_many(gpu, dim, heads, steps, slots):
         np.testing.assert_array_equal(tok, tok3[rows])
         np.testing.assert_array_equal(np.isnan(lg), np.isnan(lg3[:, rows]))
         assert np.nanmax(np.abs(lg - lg3[:, rows]), initial=0) <= 1e-5 * scale
+    eng.close()
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_depformer_few_streams_against_oracle(gpu, B):
+    """One and two streams with heads of 64, attention inside the output
+    projection for the first eight slots and a launch of its own for the ninth:
+    every step against the oracle's chain."""
+    cfg = dict(CFG, dim=512, num_heads=8, num_steps=9, kv_max_len=9, num_layers=2,
+               num_audio_emb=8)
+    w = oracle.DepformerWeights.synthetic(cfg, seed=5)
+    th, text, rand, pt, npn = _inputs(cfg, B, 31)
+    eng = sts_attn.DepthEngine(_config(cfg), _device_weights(w), max_batch=B)
+    logits = torch.empty((9, B, cfg["out_vocab"]), device="cuda")
+    tokens = eng.generate(dev(th), dev(text.view(np.int32)), 0.8, 20, 1.2, dev(rand),
+                          dev(pt.view(np.int32)), dev(npn.view(np.int32)), logits=logits)
+    agree = _check_streams(cfg, w, th, text, rand, pt, npn, host(tokens).view(np.uint32),
+                           host(logits), 20, 0.8, 1.2, range(B))
+    assert agree >= 8 * B
+    eng.close()
+
+
+def test_depformer_generate_allocates_nothing(gpu, fresh_stream):
+    """A batch whose products are large enough for the tiles of many rows: on a
+    stream without library memory the free device memory stays what it was."""
+    cfg = dict(CFG, dim=1024, num_heads=16, ffn=2816, out_vocab=2048, num_steps=1, num_layers=1,
+               kv_max_len=1, num_audio_emb=1)
+    B = 736  # x [1024, 2816] and [2048, 1024]: above 1.5e9 multiplications each
+    w = oracle.DepformerWeights.synthetic(cfg, seed=6)
+    th, text, rand, pt, npn = _inputs(cfg, B, 41)
+    eng = sts_attn.DepthEngine(_config(cfg), _device_weights(w), max_batch=B)
+    args = [dev(th), dev(text.view(np.int32)), 0.8, 20, 1.2, dev(rand), dev(pt.view(np.int32)),
+            dev(npn.view(np.int32))]
+    tokens = torch.empty((B, 1), dtype=torch.int32, device="cuda")
+    eng.generate(*args[:6], args[6], args[7], tokens=tokens)  # loads the kernels
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    eng.generate(*args[:6], args[6], args[7], tokens=tokens, stream=fresh_stream)
+    fresh_stream.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
     eng.close()
 
 
