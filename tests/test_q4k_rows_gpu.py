@@ -304,3 +304,39 @@ def test_small_weights_under_large_x(gpu, M, N, K):
     worst = (np.abs(got - ref) / size).max()
     print(f"  worst error over sum |w x|: {worst:.2e}", flush=True)
     assert worst <= 2e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 601, 1024), (2, 601, 2304), (7, 601, 1280),
+                                   (65, 11265, 2304)])
+def test_unusual_headers(gpu, M, N, K):
+    """Scales that no quantiser writes: d and dmin zero, of either sign, subnormal,
+    the largest half, an infinity or NaN; sub-block scales and mins of 0, 1 and 63.
+    Finite outputs within 2e-6 of sum |w x| (33 roundings of f32), the others as
+    the dequantised weights have them."""
+    print(f"q4k headers M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N)
+    blk = oracle._random_q4k_scaled(M + N + K, N, K).reshape(N, K // 256, 144).copy()
+    vals = np.array([0x0000, 0x8000, 0x0001, 0x83FF, 0x0400, 0x2C00, 0xAC00, 0x3C00, 0x7BFF, 0xFBFF],
+                    np.uint16)
+    for off in (0, 2):
+        blk[..., off:off + 2] = rng.choice(vals, blk.shape[:2])[..., None].view(np.uint8)
+    blk[7, 0, 0:2] = np.array([0x7C00], np.uint16).view(np.uint8)   # d = inf
+    blk[9, -1, 2:4] = np.array([0x7E00], np.uint16).view(np.uint8)  # dmin = NaN
+    blk[1::5, :, 4:16] = 0          # every scale and min 0
+    blk[2::5, :, 4:12], blk[2::5, :, 12:16] = 1, 0x11  # 1
+    blk[3::5, :, 4:16] = 0xFF       # 63
+    blk[4::5, :, 4:8] = 0           # low scales 0, mins as they are
+    x = oracle.normal(N + M, (M, K))
+    wt = torch.from_numpy(oracle.q4k_dequant(blk.reshape(-1), N, K)).cuda().double()
+    got = host(sts_attn.q4k_gemm(dev(x), sts_attn.Q4KTensor.from_q4k_bytes(blk.reshape(-1), (N, K))))
+    xd = dev(x).double()
+    ref = (xd @ wt.T.contiguous()).cpu().numpy()
+    size = (xd.abs() @ wt.abs().T.contiguous()).cpu().numpy()
+    finite = np.isfinite(ref)
+    assert not finite[:, 9].any() and not finite[:, 7].any()
+    assert finite[:, np.delete(np.arange(N), [7, 9])].all()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    assert (got[~finite & ~np.isnan(ref)] == ref[~finite & ~np.isnan(ref)]).all()
+    off = np.abs(got[finite] - ref[finite])
+    print(f"  worst error over sum |w x|: {(off / (size[finite] + 1e-300)).max():.2e}", flush=True)
+    assert (off <= 2e-6 * size[finite]).all()
