@@ -766,10 +766,10 @@ extern "C" int sts_q4k_matvec(const uint8_t* weights, const float* x, const floa
             "k = %u must be a multiple of 256 in 256..16384", k);
   STS_CHECK(aligned16(weights) && aligned16(x), "weights and x must be 16-byte aligned");
   // Several rows share the weights in the GEMM, where the matvec reads and
-  // dequantises them for each: 4 rows x [4096, 11264] 20.4 against 22.1 us, 8
-  // rows x [12288, 4096] 17 against 35, 3 rows 16.2 against 15.5; a matrix of
-  // few rows has few of the GEMM's workgroups (x [1024, 2816]: 4 rows 7.2
-  // against 5.0, 8 rows 7.4 against 8.2).
+  // dequantises them for each: 4 rows x [4096, 11264] 20.3 against 20.7 us, 8
+  // rows x [12288, 4096] 16 against 33, 3 rows 15.9 against 14.0; a matrix of
+  // few rows has few of the GEMM's workgroups (x [1024, 2816]: 4 rows 7.1
+  // against 6.4, 8 rows 7.7 against 9.7).
   if (batch >= (n < 2048 ? 8u : 4u)) {
     sts::Q4kGemmParams g;
     g.w[0] = weights;

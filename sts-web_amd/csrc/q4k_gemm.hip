@@ -557,10 +557,11 @@ struct SlotAttention {
 // where the products are a few microseconds of latency.  One wave per
 // workgroup takes RPW weight rows at once, a slot per lane (64 / RPW lanes a
 // row), R times; it stages its row of x in LDS by itself, so no barrier stands
-// in its way, and with NORM sums its squares on the way.  1 row: [3072, 1024]
-// with RMSNorm 4.0 us against 5.8 in q4k_rows_kernel, [5632, 1024] with SwiGLU
-// 4.9 against 6.9, [1024, 2816] 4.0 against about 7; [1024, 1024] 3.5, of which
-// an empty launch is 2.5.  XL: float4 of x per lane, K <= 256 XL.
+// in its way, and with NORM sums its squares on the way.  1 row, weights from
+// the last-level cache: [3072, 1024] with RMSNorm 3.3 us against 5.2 in
+// q4k_rows_kernel, [5632, 1024] with SwiGLU 4.1 against 6.3, [1024, 2816] 3.5
+// and [1024, 1024] 2.8 against 6.3 for the two, of which an empty launch is 2.5.
+// XL: float4 of x per lane, K <= 256 XL.
 //
 // ATTN: x is the output of one decode step's attention over a few slots, which
 // every wave computes for itself from q, k_new, v_new and the cache (XL float4
@@ -1237,10 +1238,10 @@ int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   const uint32_t ntiles = (nout + 15) / 16;
   const uint32_t cus = (uint32_t)device_cu_count();
   // One or two rows of x, measured against q4k_rows_kernel: 1 x [48000, 1024]
-  // 9.4 and 16.7 us, [48000, 4096] 33.3 and 47.1; 2 x [48000, 1024] 14.6 and
-  // 16.8, [48000, 2048] 28.9 and 29.1, [4096, 4096] 7.7 and 9.2.  The second row
+  // 8.2 and 15.1 us, [48000, 4096] 30.6 and 46.5; 2 x [48000, 1024] 13.1 and
+  // 14.8, [48000, 2048] 28.0 and 27.7, [4096, 4096] 6.7 and 8.8.  The second row
   // unpacks the weights again, which beyond that costs more than the 16-row
-  // tile: 2 x [16384, 3072] 20.5 and 14.1, [48000, 4096] 57.9 and 47.4.
+  // tile: 2 x [16384, 3072] 19.8 and 13.2, [48000, 4096] 56.7 and 48.2.
   if (p.K <= 4096 && (p.M == 1 || (p.M == 2 && (p.K <= 2048 || nout * p.Z <= 16 * cus)))) {
     // A wave per few weight rows; where that would be more than eight waves a
     // CU, four times the rows.
@@ -1254,14 +1255,15 @@ int launch_q4k_gemm(const Q4kGemmParams& p, hipStream_t stream) {
   // Weight tiles per workgroup: as many as bring the launch to about one
   // workgroup per CU, up to six (eight spill registers).  Every workgroup splits
   // its x rows itself, so fewer and larger workgroups split them less often:
-  // two per CU measured 12.7 against 8.1 us (64 rows x [3072, 1024]) and 28.7
-  // against 19.2 us (13 x [12288, 4096]); and waves beyond eight leave too few
-  // registers (12: 16.9 and 32.0 us).
+  // two per CU measured, with x in bf16 parts, 12.7 against 8.1 us (64 rows x
+  // [3072, 1024]) and 28.7 against 19.2 us (13 x [12288, 4096]); and waves beyond
+  // eight leave too few registers (12: 16.9 and 32.0 us).
   const uint64_t tiles = (uint64_t)ntiles * mtiles * p.Z;
   // The tiles from 33 rows on, where the products outweigh their two extra
   // launches (x split, K ranges summed): 48 rows x [12288, 4096] 37 against
-  // 50 us here, 112 x [4096, 4096] 33 against 51, but 80 x [4096, 4096] 32.5
-  // against 29.8, 32 x [12288, 4096] 34.6 against 29.7.
+  // 60 us here, 112 x [4096, 4096] 32 against 59, 512 x [22528, 4096] 256
+  // against 866, but 80 x [4096, 4096] 31.4 against 32.3, 32 x [12288, 4096]
+  // 35 against 32.
   if (p.scratch && p.M > 32 && (uint64_t)mtiles * 16 * p.N * p.K >= 1500000000ull && p.Z == 1 &&
       !p.swiglu_f && !p.norm_alpha) {
     bool done = false;
